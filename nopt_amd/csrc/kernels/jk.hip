@@ -542,6 +542,14 @@ __global__ __launch_bounds__(256) void k_syrk(const T* __restrict__ X, long ldx,
 // both triangles of J, K (ld nbf). Either output may be null. With jlive (the
 // integer Coulomb pair), J is zero in the 8-column slots (m, n/8) whose jlive
 // byte is 0: B is zero there for every Q, and the J kernels skip them.
+//
+// Bound by the latency of the partials' reads, not by their bytes: a block
+// takes 64 columns of one row (inside one exchange tile, whose edge is a
+// multiple of 64), its four waves the splits p, p + 4, p + 8, ... with eight
+// reads in flight each, and the four sums are added in the order p = 0..3, so
+// that the result is reproducible. (One thread per element over all splits,
+// one read after the other, took 32 us for the 116 partials of a 24-function
+// K and 46 us for 103 partials at 490 functions; this takes 4 and 28 us.)
 struct ItemFin {
   const double* Jpart;
   int nsj;
@@ -557,41 +565,64 @@ struct ItemFin {
   double* K;
   int gx, gy, gz;
 };
+constexpr int kFinCols = 64;
+// sum over the splits s = p, p + 4, ... < ns of src[s * stride]
+__device__ __forceinline__ double split_sum(const double* __restrict__ src, long stride, int p, int ns) {
+  double a = 0.0;
+  int s = p;
+  for (; s + 28 < ns; s += 32) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = src[(long)(s + 4 * u) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a += v[u];
+  }
+  // the last at most eight splits of this wave, read back to back as well
+  // (a split beyond the end reads the last one and counts zero)
+  double v[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = src[(long)min(s + 4 * u, ns - 1) * stride];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) a += s + 4 * u < ns ? v[u] : 0.0;
+  return a;
+}
 __device__ __forceinline__ void k_finalize_body(const VB vb, const double* __restrict__ Jpart, int nsj,
                                                 const uint8_t* __restrict__ jlive, int nsr,
                                                 const double* __restrict__ Kpart, int nsk, int ntiles, int kt,
                                                 int nbf, const int* __restrict__ perm, double* __restrict__ J,
                                                 double* __restrict__ K) {
-  const int KT = kt;  // exchange tile edge of the partials
-  const long e = (long)vb.x * blockDim.x + threadIdx.x;
-  if (e >= (long)nbf * nbf) return;
-  const int m = (int)(e / nbf), n = (int)(e % nbf);
-  if (n > m) return;
+  __shared__ double part[2][4][kFinCols];
+  const int m = vb.y, n0 = vb.x * kFinCols;
+  if (n0 > m) return;  // above the diagonal (uniform per block)
+  const int lane = threadIdx.x & 63, p = threadIdx.x >> 6, n = n0 + lane;
+  const bool ok = n <= m;
+  double sj = 0.0, sk = 0.0;
+  if (J && ok && (!jlive || jlive[(long)m * nsr + n / 8]))
+    sj = split_sum(Jpart + (long)m * nbf + n, (long)nbf * nbf, p, nsj);
+  if (K && ok) {
+    const int bi = m / kt, bj = n / kt, tile = bi * (bi + 1) / 2 + bj;
+    sk = split_sum(Kpart + ((long)tile * kt + m % kt) * kt + n % kt, (long)ntiles * kt * kt, p, nsk);
+  }
+  part[0][p][lane] = sj;
+  part[1][p][lane] = sk;
+  __syncthreads();
+  if (p > 1 || !ok) return;  // wave 0 writes J, wave 1 K
+  double* out = p == 0 ? J : K;
+  if (!out) return;
+  const double s = ((part[p][0][lane] + part[p][1][lane]) + part[p][2][lane]) + part[p][3][lane];
   // partials in the order of the integer forms (perm[new] = old)
   const long pm = perm ? perm[m] : m, pn = perm ? perm[n] : n;
-  if (J) {
-    double s = 0.0;
-    if (!jlive || jlive[(long)m * nsr + n / 8])
-      for (int k = 0; k < nsj; ++k) s += Jpart[((long)k * nbf + m) * nbf + n];
-    J[pm * nbf + pn] = s;
-    J[pn * nbf + pm] = s;
-  }
-  if (K) {
-    const int bi = m / KT, bj = n / KT;
-    const int tile = bi * (bi + 1) / 2 + bj;
-    const int r = m % KT, c = n % KT;
-    double s = 0.0;
-    for (int k = 0; k < nsk; ++k) s += Kpart[(((long)k * ntiles + tile) * KT + r) * KT + c];
-    K[pm * nbf + pn] = s;
-    K[pn * nbf + pm] = s;
-  }
+  out[pm * nbf + pn] = s;
+  out[pn * nbf + pm] = s;
 }
-__global__ void k_finalize(const double* __restrict__ Jpart, int nsj, const uint8_t* __restrict__ jlive, int nsr,
-                           const double* __restrict__ Kpart, int nsk, int ntiles, int kt, int nbf,
-                           const int* __restrict__ perm, double* __restrict__ J, double* __restrict__ K) {
+__global__ __launch_bounds__(256) void k_finalize(const double* __restrict__ Jpart, int nsj,
+                                                  const uint8_t* __restrict__ jlive, int nsr,
+                                                  const double* __restrict__ Kpart, int nsk, int ntiles, int kt,
+                                                  int nbf, const int* __restrict__ perm, double* __restrict__ J,
+                                                  double* __restrict__ K) {
   k_finalize_body(grid_vb(), Jpart, nsj, jlive, nsr, Kpart, nsk, ntiles, kt, nbf, perm, J, K);
 }
-__global__ void k_finalize_list(const ItemFin* __restrict__ items,
+__global__ __launch_bounds__(256) void k_finalize_list(const ItemFin* __restrict__ items,
     const int* __restrict__ first, int n) {
   const int i = list_item(first, n, (int)blockIdx.x);
   const ItemFin& a = items[i];
@@ -1312,7 +1343,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   // half-transform in the integer mode, or when gamma rides on it) and joined
   // before the build ends, so that they overlap the exchange.
   const bool overlap = !rec && !tm && nj > 0 && anyK;
-  const unsigned nelj = (unsigned)((nn + 255) / 256);  // finalize blocks
+  const dim3 gfin((unsigned)((nbf + kFinCols - 1) / kFinCols), (unsigned)nbf);  // output blocks
   // the integer mode works on the functions in the order of B's integer
   // forms (perm[new] = old): densities are read through it, orbitals'
   // columns too, and J, K written back through it
@@ -1342,10 +1373,10 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
                       double* J, double* K, hipStream_t st) {
     const uint8_t* jl = Jp && i8 ? c->jlive : nullptr;  // J partials of the integer pair
     if (rec)
-      rec->add(phase, kListFin, (int)nelj, 256,
-               ItemFin{Jp, nsj_, jl, c->nsr, Kp, nsk_, ntl, kt, nbf, perm, J, K, (int)nelj, 1, 1});
+      rec->add(phase, kListFin, (int)(gfin.x * gfin.y), 256,
+               ItemFin{Jp, nsj_, jl, c->nsr, Kp, nsk_, ntl, kt, nbf, perm, J, K, (int)gfin.x, (int)gfin.y, 1});
     else
-      k_finalize<<<nelj, 256, 0, st>>>(Jp, nsj_, jl, c->nsr, Kp, nsk_, ntl, kt, nbf, perm, J, K);
+      k_finalize<<<gfin, 256, 0, st>>>(Jp, nsj_, jl, c->nsr, Kp, nsk_, ntl, kt, nbf, perm, J, K);
   };
   hipStream_t sj = overlap ? c->side : s;
   auto cmark = [&](int ph) {
@@ -1517,7 +1548,6 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       pad_rows(8, w.Dp, nbf, 0, 0, it[d].K, nbf, nbf);
       continue;
     }
-    const unsigned nel = (unsigned)((nn + 255) / 256);
     if (i8) {
       // the exchange runs over the rows of the digit planes: groups of qpb
       // functions (npq of them) per segment when fused, single functions of
@@ -1559,8 +1589,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       else
         HIPCHK(nopt::launch_syrk_bf16(prec == NOPT_PREC_BF16X3 ? 2 : 3, gk, s, (const float*)w.X + off[d], ldx,
                                       nbf, naux, kpad, w.Kpart));
-      k_finalize<<<nel, 256, 0, s>>>(nullptr, 0, nullptr, 0, w.Kpart, c->nsk, c->ntiles, KT, nbf, nullptr, nullptr,
-                                     it[d].K);
+      finalize(8, nullptr, 0, w.Kpart, c->nsk, c->ntiles, KT, nullptr, it[d].K, s);
     }
     HIPCHK(hipGetLastError());
   }
