@@ -14,7 +14,7 @@ LIB = os.path.join(HERE, "libnoptjk.so")
 HOST_SRCS = ["host/basis.cpp", "host/ints.cpp", "host/errors.cpp", "host/mol_capi.cpp", "host/order.cpp"]
 # host code that calls the GPU entry points (left out of a --host-only build)
 GLUE_SRCS = ["host/ri_shim.cpp", "host/ri_cxx.cpp"]
-HIP_SRCS = ["kernels/linalg.hip", "kernels/bf16.hip", "kernels/ozaki.hip", "kernels/jk.hip"]
+HIP_SRCS = ["kernels/linalg.hip", "kernels/bf16.hip", "kernels/fp64.hip", "kernels/ozaki.hip", "kernels/jk.hip"]
 
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")

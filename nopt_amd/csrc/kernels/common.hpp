@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+typedef double d2_t __attribute__((ext_vector_type(2)));
 typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
@@ -65,6 +66,14 @@ __device__ __forceinline__ double block_sum256(double v, double* sh /* >= 4 */) 
   double r = 0.0;
   if (threadIdx.x == 0) r = sh[0] + sh[1] + sh[2] + sh[3];
   return r;
+}
+
+// row and column of the t-th tile of a lower triangle of tiles, row by row
+__device__ __forceinline__ void tri_tile(int t, int& bi, int& bj) {
+  bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
+  while (bi * (bi + 1) / 2 > t) --bi;
+  bj = t - bi * (bi + 1) / 2;
 }
 
 static inline long round_up(long x, long m) { return (x + m - 1) / m * m; }

@@ -34,6 +34,7 @@
 #include "../host/order.hpp"
 #include "common.hpp"
 #include "bf16.hpp"
+#include "fp64.hpp"
 #include "linalg.hpp"
 #include "ozaki.hpp"
 
@@ -42,7 +43,7 @@ using nopt::set_error;
 namespace {
 
 constexpr int BM = 128;     // half-transform rows per tile
-constexpr int KT = 128;     // exchange tile edge
+constexpr int KT = 128;     // exchange tile edge of the FP32 and bf16 modes
 constexpr int NSPLIT_J_MIN = 16; // minimum Q-split of the Coulomb pass
 constexpr int JCHUNK_MAX = 4096; // gamma values cached in LDS per split
 
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(256) void k_jpart(const double* __restrict__ B, lon
                                                const double* __restrict__ gamma, long gstride,
                                                double* __restrict__ Jpart, long jstride) {
   constexpr int UNR = ND == 1 ? 8 : 4;
-  __shared__ double gs[JCHUNK_MAX];  // the host keeps ND * (q1 - q0) <= JCHUNK_MAX
+  extern __shared__ double gs[];  // ND x the longest split
   const int p = blockIdx.x, s = blockIdx.y, ns = gridDim.y;
   const int q0 = (int)((long)naux * s / ns), q1 = (int)((long)naux * (s + 1) / ns);
   const int len = q1 - q0;
@@ -428,21 +429,13 @@ __global__ __launch_bounds__(256) void k_jpart(const double* __restrict__ B, lon
 }
 
 // --------------------------------------------------------------- exchange
-__device__ __forceinline__ void tri_tile(int t, int& bi, int& bj) {
-  bi = (int)((std::sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
-  while (bi * (bi + 1) / 2 > t) --bi;
-  bj = t - bi * (bi + 1) / 2;
-}
-
 // Kpart[s][tile][r][c] = sum_{Q in split s} sum_i X[Q][bi*KT+r][i] X[Q][bj*KT+c][i]
-template <typename T>
-__global__ __launch_bounds__(256) void k_syrk(const T* __restrict__ X, long ldx, int nbf, int naux,
-                                              int kpad, double* __restrict__ Kpart) {
+// (FP32 mode): FP32 chains of 16 terms, added in FP64.
+__global__ __launch_bounds__(256) void k_syrk_f32(const float* __restrict__ X, long ldx, int nbf, int naux,
+                                                  int kpad, double* __restrict__ Kpart) {
   constexpr int BK = 16;
-  using acc_t = typename std::conditional<sizeof(T) == 8, d4_t, f4_t>::type;
-  __shared__ T As[BK][KT + 2];
-  __shared__ T Bs[BK][KT + 2];
+  __shared__ float As[BK][KT + 2];
+  __shared__ float Bs[BK][KT + 2];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int wr = w >> 1, wc = w & 1;
   int bi, bj;
@@ -451,26 +444,26 @@ __global__ __launch_bounds__(256) void k_syrk(const T* __restrict__ X, long ldx,
   const int q0 = (int)((long)naux * s / ns), q1 = (int)((long)naux * (s + 1) / ns);
   const int r = t >> 1, kk = (t & 1) * 8;
   const bool ra = bi * KT + r < nbf, rb = bj * KT + r < nbf;
-  acc_t acc[4][4];
-  d4_t acc64[4][4];  // used by the FP32 variant only
+  f4_t acc[4][4];
+  d4_t acc64[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      acc[i][j] = acc_t{0, 0, 0, 0};
+      acc[i][j] = f4_t{0, 0, 0, 0};
       acc64[i][j] = d4_t{0, 0, 0, 0};
     }
-  T a_reg[8], b_reg[8];
+  float a_reg[8], b_reg[8];
   auto gload = [&](int q, int i0) {
-    const T* xa = X + ((long)q * nbf + bi * KT + r) * ldx + i0 + kk;
-    const T* xb = X + ((long)q * nbf + bj * KT + r) * ldx + i0 + kk;
+    const float* xa = X + ((long)q * nbf + bi * KT + r) * ldx + i0 + kk;
+    const float* xb = X + ((long)q * nbf + bj * KT + r) * ldx + i0 + kk;
     if (ra)
-      load8<T>(xa, a_reg);
+      load8<float>(xa, a_reg);
     else
 #pragma unroll
       for (int i = 0; i < 8; ++i) a_reg[i] = 0;
     if (rb)
-      load8<T>(xb, b_reg);
+      load8<float>(xb, b_reg);
     else
 #pragma unroll
       for (int i = 0; i < 8; ++i) b_reg[i] = 0;
@@ -493,7 +486,7 @@ __global__ __launch_bounds__(256) void k_syrk(const T* __restrict__ X, long ldx,
       if (nq < q1) gload(nq, ni);
 #pragma unroll
       for (int ks = 0; ks < BK; ks += 4) {
-        T a[4], b[4];
+        float a[4], b[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = As[ks + lane / 16][wr * 64 + i * 16 + lane % 16];
 #pragma unroll
@@ -501,24 +494,16 @@ __global__ __launch_bounds__(256) void k_syrk(const T* __restrict__ X, long ldx,
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            if constexpr (sizeof(T) == 8)
-              acc[i][j] = mfma_f64(a[i], b[j], acc[i][j]);
-            else
-              acc[i][j] = mfma_f32(a[i], b[j], acc[i][j]);
-          }
+          for (int j = 0; j < 4; ++j) acc[i][j] = mfma_f32(a[i], b[j], acc[i][j]);
       }
-      if constexpr (sizeof(T) == 4) {
-        // FP32 chains of BK terms, accumulated in FP64
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < 4; ++j) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc64[i][j][v] += (double)acc[i][j][v];
-            acc[i][j] = acc_t{0, 0, 0, 0};
-          }
-      }
+          for (int v = 0; v < 4; ++v) acc64[i][j][v] += (double)acc[i][j][v];
+          acc[i][j] = f4_t{0, 0, 0, 0};
+        }
     }
   }
   double* Kt = Kpart + ((long)s * gridDim.x + blockIdx.x) * KT * KT;
@@ -527,14 +512,8 @@ __global__ __launch_bounds__(256) void k_syrk(const T* __restrict__ X, long ldx,
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int rr = wr * 64 + i * 16 + acc_row<T>(lane, v);
-        const int cc = wc * 64 + j * 16 + lane % 16;
-        if constexpr (sizeof(T) == 4)
-          Kt[rr * KT + cc] = acc64[i][j][v];
-        else
-          Kt[rr * KT + cc] = acc[i][j][v];
-      }
+      for (int v = 0; v < 4; ++v)
+        Kt[(wr * 64 + i * 16 + acc_row<float>(lane, v)) * KT + wc * 64 + j * 16 + lane % 16] = acc64[i][j][v];
 }
 
 // --------------------------------------------------------------- finalize
@@ -733,7 +712,10 @@ struct nopt_jk_ctx {
   size_t Xd_bytes = 0;
   void* Xe = nullptr;
   size_t Xe_bytes = 0;
-  int ntiles8 = 0, nsk8 = 0;  // 64x64 exchange tiles of the integer path
+  int ntiles8 = 0, nsk8 = 0;  // 64x64 exchange tiles of the FP64 and integer paths; the integer path's Q-splits
+  // Q-splits of the FP32 and bf16 exchanges: as many blocks of their 128x128
+  // tiles as the FP64 exchange has of its own
+  int nsk128() const { return (int)std::max(1L, std::min(naux, (long)nsk * ntiles8 / ntiles)); }
   // the lower triangle of B as packed rows in 16-column segments (N28 as
   // int32, then d4 as bytes: 5*splane bytes), read by the Coulomb pair and,
   // without bfull, by the half-transform; the segment and slot tables, gamma
@@ -1323,8 +1305,9 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   // density; a recorded build runs every exchange before any K output, so
   // there each segment of the batch has its own range
   const int kranges = rec ? std::max(nxs, 1) : segs_max;
-  wb.Kpart = sizeof(double) * (i8 ? (size_t)kranges * c->nsk8 * c->ntiles8 * nopt::kSyrkI8Tile * nopt::kSyrkI8Tile
-                                  : (size_t)c->nsk * c->ntiles * KT * KT);
+  wb.Kpart = sizeof(double) * (i8    ? (size_t)kranges * c->nsk8 * c->ntiles8 * nopt::kSyrkI8Tile * nopt::kSyrkI8Tile
+                               : f64 ? (size_t)c->nsk * c->ntiles8 * nopt::kSyrkF64Tile * nopt::kSyrkF64Tile
+                                     : (size_t)c->nsk128() * c->ntiles * KT * KT);
   if (nj) wb.Jpart = sizeof(double) * nj * nsj * nn;
   wb.Dp = sizeof(double) * std::max(nj, 1) * c->dstride;
   wb.gamma = sizeof(double) * std::max(nj, 1) * naux;
@@ -1419,9 +1402,10 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       return nopt::launch_jpart_slots(nj, nsj, sj, c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lslots,
                                       c->nlslots, c->lsegs, c->nlseg, w.gamma, naux, Jpart, (long)nsj * nn);
     dim3 gj((nbf + 1) / 2, nsj);
+    const size_t jlds = sizeof(double) * nj * ((naux + nsj - 1) / nsj);  // at most JCHUNK_MAX values
 #define NOPT_JP(ND)                                                                                     \
   case ND:                                                                                              \
-    k_jpart<ND><<<gj, 256, 0, sj>>>(c->B64, c->ld64, nbf, naux, w.gamma, naux, Jpart, (long)nsj * nn); \
+    k_jpart<ND><<<gj, 256, jlds, sj>>>(c->B64, c->ld64, nbf, naux, w.gamma, naux, Jpart, (long)nsj * nn); \
     break;
     switch (nj) { NOPT_JP(1) NOPT_JP(2) NOPT_JP(3) NOPT_JP(4) }
 #undef NOPT_JP
@@ -1581,15 +1565,17 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       finalize(8, nullptr, 0, w.Kpart + kfirst * kseg, nsum * c->nsk8, c->ntiles8, nopt::kSyrkI8Tile, nullptr,
                it[d].K, s);
     } else {
-      dim3 gk(c->ntiles, c->nsk);
+      const int ns = f64 ? nopt::syrk_f64_splits(c->nsk, naux, kpad) : c->nsk128();
+      const int ntl = f64 ? c->ntiles8 : c->ntiles;
+      dim3 gk(ntl, ns);
       if (f64)
-        k_syrk<double><<<gk, 256, 0, s>>>((const double*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart);
+        HIPCHK(nopt::launch_syrk_f64(ntl, ns, s, (const double*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart));
       else if (prec == NOPT_PREC_FP32)
-        k_syrk<float><<<gk, 256, 0, s>>>((const float*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart);
+        k_syrk_f32<<<gk, 256, 0, s>>>((const float*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart);
       else
         HIPCHK(nopt::launch_syrk_bf16(prec == NOPT_PREC_BF16X3 ? 2 : 3, gk, s, (const float*)w.X + off[d], ldx,
                                       nbf, naux, kpad, w.Kpart));
-      finalize(8, nullptr, 0, w.Kpart, c->nsk, c->ntiles, KT, nullptr, it[d].K, s);
+      finalize(8, nullptr, 0, w.Kpart, ns, ntl, f64 ? nopt::kSyrkF64Tile : KT, nullptr, it[d].K, s);
     }
     HIPCHK(hipGetLastError());
   }
@@ -1690,7 +1676,6 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
   c->mtiles64 = (int)((nbf + 63) / 64);
   c->ktn = (int)((nbf + KT - 1) / KT);
   c->ntiles = c->ktn * (c->ktn + 1) / 2;
-  c->nsk = std::max(1, std::min((int)naux, (1024 + c->ntiles - 1) / c->ntiles));
   {
     // integer exchange: by default Q-splits in multiples of 8 (as many
     // blocks on every XCD), sized so that the blocks of an XCD fill whole
@@ -1700,6 +1685,8 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || ncu <= 0)
       ncu = 256;
+    // FP64 exchange: four blocks per CU fit, one round of them
+    c->nsk = (int)std::max(1L, std::min(naux, 4L * ncu / c->ntiles8));
     const long slots = 2L * ncu / 8;  // per XCD
     int best = 8;
     double best_eff = 0.0;
@@ -1729,8 +1716,10 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
   if (!rc) rc = dev_alloc((void**)&c->gpart, sizeof(double) * naux * c->mtiles64, "gamma partials");
   if (!rc) rc = dev_alloc((void**)&c->gamma, sizeof(double) * kMaxBatch * naux, "gamma");
   if (!rc) {
-    c->Kpart_bytes = sizeof(double) * std::max((long)c->nsk * c->ntiles * KT * KT,
-                                               (long)c->nsk8 * c->ntiles8 * nopt::kSyrkI8Tile * nopt::kSyrkI8Tile);
+    static_assert(nopt::kSyrkI8Tile == nopt::kSyrkF64Tile, "ntiles8 counts the tiles of both");
+    c->Kpart_bytes = sizeof(double) * std::max((long)c->nsk128() * c->ntiles * KT * KT,
+                                               (long)std::max(c->nsk, c->nsk8) * c->ntiles8 * nopt::kSyrkI8Tile *
+                                                   nopt::kSyrkI8Tile);
     rc = dev_alloc((void**)&c->Kpart, c->Kpart_bytes, "K partials");
   }
   c->dstride = nbf * std::max(c->ld64, c->ld8);

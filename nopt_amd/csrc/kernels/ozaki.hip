@@ -1210,13 +1210,6 @@ __global__ __launch_bounds__(256) void k_jpart_slots_list(const ItemJ* __restric
 
 
 // ------------------------------------------------------------------ exchange
-__device__ __forceinline__ void tri_tile(int t, int& bi, int& bj) {
-  bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
-  while (bi * (bi + 1) / 2 > t) --bi;
-  bj = t - bi * (bi + 1) / 2;
-}
-
 // Kpart[s][tile][r][c] = sum_{Q in split s} 2^(e_Qm + e_Qn - 12) sum_{k+l<=4}
 //   2^(-7(k+l)) <Xd_k[Q][m][:], Xd_l[Q][n][:]>,  m = 64 bi + r, n = 64 bj + c,
 // k, l < 4 (13 digit pairs in 5 exact int32 classes, combined in FP64 once
