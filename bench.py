@@ -76,9 +76,9 @@ def time_builds(ctx, dD, dC, nocc, dJ, dK, prec, steps, warmup, synchronize, tim
 
 # kernels of each timed phase, per mode
 KERNELS = {
-    "half_transform": {"fp64": "k_half<double, 6>", "fp32": "k_half<float, 6>", "bf16x6": "k_half_bf16<3, 6>",
+    "half_transform": {"fp64": "k_half_f64<6, 1, 2>", "fp32": "k_half_f32<6>", "bf16x6": "k_half_bf16<3, 6>",
                        "bf16x3": "k_half_bf16<2, 6>", "int8": "k_half_i8<6, 2, 4, 2, 32, 4, false>"},
-    "gamma": {"fp64": "k_gamma (fused partials)", "fp32": "k_gamma (fused partials)",
+    "gamma": {"fp64": "none (the J kernel adds the fused partials)", "fp32": "k_gamma (fused partials)",
               "bf16x6": "k_gamma (fused partials)", "bf16x3": "k_gamma (fused partials)",
               "int8": "k_gamma_slots<1, 2, true>"},
     "coulomb_j": {"fp64": "k_jpart<1>", "fp32": "k_jpart<1>", "bf16x6": "k_jpart<1>", "bf16x3": "k_jpart<1>",

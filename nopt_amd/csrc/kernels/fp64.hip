@@ -10,6 +10,167 @@
 namespace nopt {
 namespace {
 
+// ------------------------------------------------------------ half-transform
+// X[r][c] = sum_n B[r][n] C[c][n] over the rows r = Q*nbf + m of all functions
+// as one range (no padding of the rows of a function), and with ND > 0 the
+// partial sums of gamma_d[Q] = sum_mn B[Q][m][n] D_d[m][n].
+//
+// A block takes 128 rows and 16 NT columns, a wave 32 rows of them. Only C
+// passes through LDS (all four waves read it; slabs of 16, double buffered,
+// one barrier per slab of 16 NT products per wave); a wave's rows of B go
+// straight from global memory to its registers, a row's 16 values of a slab in
+// two loads back to back, so that the second finds its line in the L1, and are
+// requested again for the next slab as soon as their products are issued. The
+// rows of D follow those of B. The order of the terms is free: in a step of
+// eight, lane l holds the terms 2 (l / 16) and 2 (l / 16) + 1 of row l % 16 of
+// either operand, the first for one product, the second for the next.
+//
+// At C20H42 (490 functions, 2366 auxiliary functions, 81 orbitals, one
+// density) 1.80 ms, 51 TFLOP/s of useful products (61 as issued: 96 columns),
+// against 2.85 ms with B and C staged through LDS by loads of 64-byte lane
+// stride in 128-row tiles per function; 1.69 ms without the density, whose rows
+// cost registers (two waves per SIMD instead of three). With up to three
+// column tiles it runs at the rate of B's reads (1.0-1.1 ms here). One row of
+// D per function of four waves through LDS, extra columns by vector
+// instructions and wave tiles of 16, 48 or 64 rows were slower.
+//
+// The column groups of a row tile are consecutive blocks of one XCD, so that
+// the second finds B in its L2. gpart[d*gstride + tile + Q] is the part of
+// gamma_d[Q] in row tile `tile` (consecutive (tile, Q) pairs that share rows
+// have consecutive sums tile + Q).
+constexpr int kHalfRows = kHalfF64Rows;
+template <int NT, int ND, int OCC>
+__global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict__ B, long ld, long rows, int nbf,
+                                                       const double* __restrict__ Cp, const double* __restrict__ Dp,
+                                                       long dstride, double* __restrict__ X, int ldx,
+                                                       double* __restrict__ gpart, long gstride, int ntile,
+                                                       int groups) {
+  constexpr int MI = 2, NC = 16 * NT, CPT = (NC * 8 + 255) / 256;
+  __shared__ __attribute__((aligned(16))) double sm[2][NC][18];
+  const int t = threadIdx.x, lane = t & 63, lr = lane & 15, g = lane >> 4, w = t >> 6;
+  const int local = blockIdx.x / 8, cg = local % groups, tile = (local / groups) * 8 + (int)(blockIdx.x % 8);
+  if (tile >= ntile) return;
+  const long rb = (long)tile * kHalfRows;  // the block's first row
+  const char* Bb = reinterpret_cast<const char*>(B + rb * ld);
+  const char* Db = reinterpret_cast<const char*>(Dp);
+  const char* Cb = reinterpret_cast<const char*>(Cp);
+  // byte offsets of the lane's rows (beyond the last row: that row again, not written)
+  unsigned ao[MI], dof[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int r = (int)min((long)((w * MI + i) * 16 + lr), rows - 1 - rb);
+    ao[i] = 8u * (unsigned)(r * (int)ld + 2 * g);
+    dof[i] = 8u * (unsigned)((int)((rb + r) % nbf) * (int)ld + 2 * g);
+  }
+  // C loader: 16-byte chunk e % 8 of column e / 8 (a column beyond ldx repeats the last one, not written)
+  unsigned co[CPT];
+#pragma unroll
+  for (int u = 0; u < CPT; ++u) {
+    const int e = min(t + 256 * u, NC * 8 - 1);
+    co[u] = 8u * (unsigned)(min(cg * NC + (e >> 3), ldx - 1) * (int)ld + 2 * (e & 7));
+  }
+  d2_t a[MI][2], d[ND ? MI : 1][ND ? ND : 1][2], cr[CPT];
+  auto aload = [&](int i, long k) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      a[i][h] = *reinterpret_cast<const d2_t*>(Bb + 8 * k + ao[i] + 64 * h);
+#pragma unroll
+      for (int q = 0; q < ND; ++q)
+        d[i][q][h] = *reinterpret_cast<const d2_t*>(Db + 8 * (q * dstride + k) + dof[i] + 64 * h);
+    }
+  };
+  auto cload = [&](long k) {
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) cr[u] = *reinterpret_cast<const d2_t*>(Cb + 8 * k + co[u]);
+  };
+  auto cstore = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+      const int e = t + 256 * u;
+      if ((u + 1) * 256 <= NC * 8 || e < NC * 8) *reinterpret_cast<d2_t*>(&sm[buf][e >> 3][2 * (e & 7)]) = cr[u];
+    }
+  };
+  d4_t acc[MI][NT];
+  double rd[MI][ND ? ND : 1];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = d4_t{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < ND; ++q) rd[i][q] = 0.0;
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i) aload(i, 0);
+  cload(0);
+  cstore(0);
+  __syncthreads();
+  int cur = 0;
+  for (int k0 = 0; k0 < nbf; k0 += 16, cur ^= 1) {
+    const int kn = k0 + 16 < nbf ? k0 + 16 : k0;  // the last slab again, unused, after the last
+    cload(kn);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        d2_t cc[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) cc[j] = *reinterpret_cast<const d2_t*>(&sm[cur][j * 16 + lr][8 * h + 2 * g]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i][j] = mfma_f64(a[i][h][e], cc[j][e], acc[i][j]);
+#pragma unroll
+        for (int q = 0; q < ND; ++q)
+          rd[i][q] = fma(a[i][h][1], d[i][q][h][1], fma(a[i][h][0], d[i][q][h][0], rd[i][q]));
+      }
+      aload(i, kn);
+      // keeps the operand reads of the next rows, and their registers, behind these products
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cstore(cur ^ 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const long r = rb + (w * MI + i) * 16 + acc_row<double>(lane, v);
+      if (r < rows) {
+        double* xr = X + r * ldx + cg * NC;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          if (cg * NC + j * 16 + lr < ldx) xr[j * 16 + lr] = acc[i][j][v];
+      }
+    }
+  if constexpr (ND > 0) {
+    if (cg != 0) return;
+    double(*red)[kHalfRows] = reinterpret_cast<double(*)[kHalfRows]>(&sm[0][0][0]);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int q = 0; q < ND; ++q) {
+        double x = rd[i][q];
+        x += __shfl_xor(x, 16, 64);
+        x += __shfl_xor(x, 32, 64);
+        if (g == 0) red[q][(w * MI + i) * 16 + lr] = x;
+      }
+    __syncthreads();
+    // a wave per function: its rows inside the tile
+    const long re = min(rb + kHalfRows, rows);
+    const int Q0 = (int)(rb / nbf), Q1 = (int)((re - 1) / nbf);
+    for (int Q = Q0 + w; Q <= Q1; Q += 4) {
+      const int lo = (int)(max((long)Q * nbf, rb) - rb), hi = (int)(min((long)(Q + 1) * nbf, re) - rb);
+#pragma unroll
+      for (int q = 0; q < ND; ++q) {
+        double x = 0.0;
+        for (int r = lane; r < kHalfRows; r += 64) x += r >= lo && r < hi ? red[q][r] : 0.0;
+        x = warp_sum(x);
+        if (lane == 0) gpart[q * gstride + tile + Q] = x;
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ exchange
 // Tiles of 64 x 64 with four waves of 32 x 32, four blocks per CU. The
 // contraction runs over (Q, orbital) as one index, kpad orbitals per function
@@ -124,6 +285,39 @@ __global__ __launch_bounds__(256, 4) void k_syrk_f64(const double* __restrict__ 
 }
 
 }  // namespace
+
+int half_f64_nt(long ncol, int* groups) {
+  const int t = (int)std::max(1L, (ncol + 15) / 16);
+  *groups = (t + 7) / 8;
+  return (t + *groups - 1) / *groups;
+}
+
+hipError_t launch_half_f64(int nt, int groups, int nd, hipStream_t s, const double* B, long ld, int naux, int nbf,
+                           const double* Cp, const double* Dp, long dstride, double* X, long ldx, double* gpart) {
+  const long rows = (long)naux * nbf;
+  const int ntile = half_f64_tiles(naux, nbf);
+  if (nd < 0 || nd > kHalfF64Dens || groups < 1 || 16L * nt * groups < ldx || 16L * nt * (groups - 1) >= ldx ||
+      ldx % 2 || ld % 16 || ld < nbf || (nd && (!Dp || !gpart)) || ld * std::max(ldx, (long)kHalfF64Rows) > 1L << 28 ||
+      ld * nbf > 1L << 28)
+    return hipErrorInvalidValue;
+  const unsigned grid = (unsigned)((ntile + 7) / 8 * 8 * groups);
+#define NOPT_HALF_F64(NT_, ND_)                                                                                  \
+  if (nt == NT_ && nd == ND_)                                                                                    \
+    k_half_f64<NT_, ND_, (NT_ <= 4 && ND_ < 2 ? 3 : 2)><<<grid, 256, 0, s>>>(B, ld, rows, nbf, Cp, Dp, dstride, X, (int)ldx, \
+                                                                 gpart, half_f64_gstride(naux, nbf), ntile, groups);
+#define NOPT_HALF_F64_ND(NT_) NOPT_HALF_F64(NT_, 0) NOPT_HALF_F64(NT_, 1) NOPT_HALF_F64(NT_, 2)
+  NOPT_HALF_F64_ND(1)
+  NOPT_HALF_F64_ND(2)
+  NOPT_HALF_F64_ND(3)
+  NOPT_HALF_F64_ND(4)
+  NOPT_HALF_F64_ND(5)
+  NOPT_HALF_F64_ND(6)
+  NOPT_HALF_F64_ND(7)
+  NOPT_HALF_F64_ND(8)
+#undef NOPT_HALF_F64_ND
+#undef NOPT_HALF_F64
+  return nt < 1 || nt > 8 ? hipErrorInvalidValue : hipGetLastError();
+}
 
 int syrk_f64_splits(int nsplit, int naux, int kpad) {
   return (int)std::max(1L, std::min((long)nsplit, (long)naux * kpad / 32));

@@ -1,10 +1,26 @@
-// FP64 exchange on the matrix cores (see fp64.hip).
+// FP64 half-transform and exchange on the matrix cores (see fp64.hip).
 #pragma once
 #include "common.hpp"
 
 #include <algorithm>
 
 namespace nopt {
+// X[r*ldx + c] = sum_n B[r*ld + n] Cp[c*ld + n] for the rows r = Q*nbf + m of
+// all naux functions and c < ldx (an even count; column groups of 16 nt,
+// half_f64_nt picks nt and their number), B's and Cp's columns nbf.. up to the
+// next multiple of 16 zero. With nd > 0 also the gamma partials of the nd
+// densities Dp + d*dstride (rows of ld): those of gamma_d[Q] are
+// gpart[d*gstride + tile + Q] for the tiles of kHalfF64Rows rows that hold
+// rows of Q, tile = Q*nbf / kHalfF64Rows .. (Q*nbf + nbf - 1) / kHalfF64Rows.
+constexpr int kHalfF64Rows = 128, kHalfF64Dens = 2;
+static inline int half_f64_tiles(long naux, long nbf) {
+  return (int)((naux * nbf + kHalfF64Rows - 1) / kHalfF64Rows);
+}
+static inline long half_f64_gstride(long naux, long nbf) { return half_f64_tiles(naux, nbf) + naux; }
+int half_f64_nt(long ncol, int* groups);
+hipError_t launch_half_f64(int nt, int groups, int nd, hipStream_t s, const double* B, long ld, int naux, int nbf,
+                           const double* Cp, const double* Dp, long dstride, double* X, long ldx, double* gpart);
+
 constexpr int kSyrkF64Tile = 64;  // exchange tile edge
 
 // Kpart[split][tile][r][c] = sum over the split's functions Q of

@@ -42,7 +42,7 @@ using nopt::set_error;
 
 namespace {
 
-constexpr int BM = 128;     // half-transform rows per tile
+constexpr int BM = 128;     // half-transform rows per tile (FP32 and bf16 modes)
 constexpr int KT = 128;     // exchange tile edge of the FP32 and bf16 modes
 constexpr int NSPLIT_J_MIN = 16; // minimum Q-split of the Coulomb pass
 constexpr int JCHUNK_MAX = 4096; // gamma values cached in LDS per split
@@ -162,14 +162,9 @@ __global__ void k_pad_copy_list(const ItemPad* __restrict__ items, const int* __
                           a.ldd, a.rows_pad, a.rperm, a.cperm);
 }
 
-// --------------------------------------------------- half-transform f64/f32
+// ---------------------------------------------------- half-transform (FP32)
 // X[Q][m][col] = sum_n B[Q][m][n] Cp[col][n] for one (m-tile, Q, column group)
 // and gpart[Q][mtile] = sum over the tile of B[Q][m][n] D[m][n].
-template <typename T>
-struct Vec8 {
-  T v[8];
-};
-
 template <typename T>
 __device__ __forceinline__ void load8(const T* p, T* out) {
   if constexpr (sizeof(T) == 8) {
@@ -193,17 +188,17 @@ __device__ __forceinline__ void load8(const T* p, T* out) {
   }
 }
 
-// B is always read in FP64; the FP32 variant rounds it while staging into LDS,
-// so the fused gamma partials are FP64 in both variants.
-template <typename T, int NT>
-__global__ __launch_bounds__(256) void k_half(const double* __restrict__ B, long ld, int nbf,
-                                              const T* __restrict__ Cp, const double* __restrict__ Dp,
-                                              T* __restrict__ X, long ldx, double* __restrict__ gpart,
-                                              int mtiles) {
+// FP32 mode: B is read in FP64 and rounded while staging into LDS, so the
+// fused gamma partials are FP64; FP32 chains of 16 terms (rounded to nearest by
+// the matrix unit), added across chains in FP64.
+template <int NT>
+__global__ __launch_bounds__(256) void k_half_f32(const double* __restrict__ B, long ld, int nbf,
+                                                  const float* __restrict__ Cp, const double* __restrict__ Dp,
+                                                  float* __restrict__ X, long ldx, double* __restrict__ gpart,
+                                                  int mtiles) {
   constexpr int BN = 16 * NT, BK = 16;
-  using acc_t = typename std::conditional<sizeof(T) == 8, d4_t, f4_t>::type;
-  __shared__ T As[BK][BM + 2];
-  __shared__ T Cs[BK][BN + 2];
+  __shared__ float As[BK][BM + 2];
+  __shared__ float Cs[BK][BN + 2];
   __shared__ double red[4];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int mtile = blockIdx.x;
@@ -215,30 +210,24 @@ __global__ __launch_bounds__(256) void k_half(const double* __restrict__ B, long
   const double* Arow = B + ((long)Q * nbf + m0 + ar) * ld + ak;
   const double* Drow = Dp + (long)(m0 + ar) * ld + ak;
   const bool c_ok = t < 2 * BN;
-  const T* Crow = Cp + ((long)cg * BN + (t >> 1)) * ld + ak;
-  acc_t acc[2][NT];
-  d4_t acc64[2][NT];  // used by the FP32 variant only
+  const float* Crow = Cp + ((long)cg * BN + (t >> 1)) * ld + ak;
+  f4_t acc[2][NT];
+  d4_t acc64[2][NT];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      acc[i][j] = acc_t{0, 0, 0, 0};
+      acc[i][j] = f4_t{0, 0, 0, 0};
       acc64[i][j] = d4_t{0, 0, 0, 0};
     }
   double rd = 0.0;
   double a_reg[8];
-  T c_reg[8];
+  float c_reg[8];
   double d_reg[8];
   auto gload = [&](int k0) {
     if (arow_ok) {
       load8<double>(Arow + k0, a_reg);
-      const double2* dq = reinterpret_cast<const double2*>(Drow + k0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        double2 x = dq[i];
-        d_reg[2 * i] = x.x;
-        d_reg[2 * i + 1] = x.y;
-      }
+      load8<double>(Drow + k0, d_reg);
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -246,14 +235,14 @@ __global__ __launch_bounds__(256) void k_half(const double* __restrict__ B, long
         d_reg[i] = 0;
       }
     }
-    if (c_ok) load8<T>(Crow + k0, c_reg);
+    if (c_ok) load8<float>(Crow + k0, c_reg);
   };
   gload(0);
   for (int k0 = 0; k0 < ld; k0 += BK) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      As[ak + i][ar] = (T)a_reg[i];
+      As[ak + i][ar] = (float)a_reg[i];
       rd += a_reg[i] * d_reg[i];
     }
     if (c_ok) {
@@ -264,7 +253,7 @@ __global__ __launch_bounds__(256) void k_half(const double* __restrict__ B, long
     if (k0 + BK < ld) gload(k0 + BK);
 #pragma unroll
     for (int ks = 0; ks < BK; ks += 4) {
-      T a[2], b[NT];
+      float a[2], b[NT];
 #pragma unroll
       for (int i = 0; i < 2; ++i) a[i] = As[ks + lane / 16][w * 32 + i * 16 + lane % 16];
 #pragma unroll
@@ -272,40 +261,26 @@ __global__ __launch_bounds__(256) void k_half(const double* __restrict__ B, long
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          if constexpr (sizeof(T) == 8)
-            acc[i][j] = mfma_f64(a[i], b[j], acc[i][j]);
-          else
-            acc[i][j] = mfma_f32(a[i], b[j], acc[i][j]);
-        }
+        for (int j = 0; j < NT; ++j) acc[i][j] = mfma_f32(a[i], b[j], acc[i][j]);
     }
-    if constexpr (sizeof(T) == 4) {
-      // FP32 chains of BK terms (rounded to nearest by the MFMA), accumulated
-      // across chains in FP64
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
+      for (int j = 0; j < NT; ++j) {
 #pragma unroll
-          for (int v = 0; v < 4; ++v) acc64[i][j][v] += (double)acc[i][j][v];
-          acc[i][j] = acc_t{0, 0, 0, 0};
-        }
-    }
+        for (int v = 0; v < 4; ++v) acc64[i][j][v] += (double)acc[i][j][v];
+        acc[i][j] = f4_t{0, 0, 0, 0};
+      }
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int m = m0 + w * 32 + i * 16 + acc_row<T>(lane, v);
+      const int m = m0 + w * 32 + i * 16 + acc_row<float>(lane, v);
       if (m < nbf) {
-        T* xr = X + ((long)Q * nbf + m) * ldx + (long)cg * BN + lane % 16;
+        float* xr = X + ((long)Q * nbf + m) * ldx + (long)cg * BN + lane % 16;
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          if constexpr (sizeof(T) == 4)
-            xr[j * 16] = (T)acc64[i][j][v];
-          else
-            xr[j * 16] = acc[i][j][v];
-        }
+        for (int j = 0; j < NT; ++j) xr[j * 16] = (float)acc64[i][j][v];
       }
     }
   if (cg == 0) {
@@ -371,10 +346,11 @@ __global__ void k_gamma(const double* __restrict__ gpart, int mtiles, int naux,
 // pair (p, nbf-1-p): nbf+1 elements, read as aligned pairs of columns (a
 // row's last pair may include its first upper element, which lies inside the
 // row because ld > nbf and is not written). The Q loop is unrolled so that UNR
-// loads per thread are in flight.
+// loads per thread are in flight. gamma[d*gstride + Q], or with grows > 0 its
+// partials as the FP64 half-transform leaves them (launch_half_f64).
 template <int ND>
 __global__ __launch_bounds__(256) void k_jpart(const double* __restrict__ B, long ld, int nbf, int naux,
-                                               const double* __restrict__ gamma, long gstride,
+                                               const double* __restrict__ gamma, long gstride, int grows,
                                                double* __restrict__ Jpart, long jstride) {
   constexpr int UNR = ND == 1 ? 8 : 4;
   extern __shared__ double gs[];  // ND x the longest split
@@ -383,7 +359,19 @@ __global__ __launch_bounds__(256) void k_jpart(const double* __restrict__ B, lon
   const int len = q1 - q0;
   for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x)
 #pragma unroll
-    for (int d = 0; d < ND; ++d) gs[d * len + q - q0] = gamma[d * gstride + q];
+    for (int d = 0; d < ND; ++d) {
+      const double* gd = gamma + d * gstride + q;
+      double v = 0.0;
+      if (grows > 0) {  // partials of the FP64 half-transform: one per tile of grows rows that holds rows of q
+        const long r = (long)q * nbf;
+        const int t1 = (int)((r + nbf - 1) / grows);
+#pragma unroll 4
+        for (int tl = (int)(r / grows); tl <= t1; ++tl) v += gd[tl];
+      } else {
+        v = gd[0];
+      }
+      gs[d * len + q - q0] = v;
+    }
   __syncthreads();
   auto g = [&](int d, int i) { return gs[d * len + i]; };
   const int m1 = p, m2 = nbf - 1 - p;
@@ -849,12 +837,11 @@ int nt_for(long nocc, int* ngroups) {
   return nt;
 }
 
-template <typename T>
-hipError_t launch_half(int nt, dim3 grid, hipStream_t s, const double* B, long ld, int nbf, const T* Cp,
-                       const double* Dp, T* X, long ldx, double* gpart, int mtiles) {
+hipError_t launch_half_f32(int nt, dim3 grid, hipStream_t s, const double* B, long ld, int nbf, const float* Cp,
+                           const double* Dp, float* X, long ldx, double* gpart, int mtiles) {
 #define NOPT_HALF(NTV) \
   case NTV:            \
-    k_half<T, NTV><<<grid, 256, 0, s>>>(B, ld, nbf, Cp, Dp, X, ldx, gpart, mtiles); \
+    k_half_f32<NTV><<<grid, 256, 0, s>>>(B, ld, nbf, Cp, Dp, X, ldx, gpart, mtiles); \
     break;
   switch (nt) {
     NOPT_HALF(1)
@@ -1212,7 +1199,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     return set_error(NOPT_ESTATE, "the context keeps no integer form of B (NOPT_CTX_FP64_ONLY): integer mode unavailable");
   if (!i8 && !c->B64)
     return set_error(NOPT_ESTATE, "the context keeps no FP64 B (NOPT_CTX_INT8_ONLY): only the integer mode is available");
-  const long unit = bf ? 32 : 16;  // column padding of each orbital block
+  const long unit = f64 ? 4 : bf ? 32 : 16;  // column padding of each orbital block
   long off[kMaxBatch + 1];
   int jl[kMaxBatch];
   int nj = 0;
@@ -1228,12 +1215,14 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   }
   const long ncol = off[nd];
   const bool anyK = ncol > 0;
-  // one density with J and K in a non-integer mode: gamma rides on the
-  // half-transform (row dots of the B panels already in registers)
-  const bool fused = !i8 && nd == 1 && nj == 1 && anyK;
+  // one density with J and K in a non-integer mode (up to two in FP64): gamma
+  // rides on the half-transform (row dots of the B panels already in registers)
+  const bool fused = !i8 && anyK && (f64 ? nj >= 1 && nj <= nopt::kHalfF64Dens : nd == 1 && nj == 1);
   int ngroups = 1;
-  const int nt = i8 ? nt_for_i8(anyK ? ncol : 1, &ngroups) : nt_for(anyK ? ncol : 1, &ngroups);
-  const long ldx = (long)nt * 16 * ngroups;  // stacked, padded orbital count
+  const int nt = i8    ? nt_for_i8(anyK ? ncol : 1, &ngroups)
+                 : f64 ? nopt::half_f64_nt(ncol, &ngroups)
+                       : nt_for(anyK ? ncol : 1, &ngroups);
+  const long ldx = f64 && anyK ? ncol : (long)nt * 16 * ngroups;  // stacked, padded orbital count
   const long ldb = i8 ? c->ld8 : c->ld64;    // leading dimension of the staged D and C
   const int mt = i8 ? c->mtiles64 : c->mtiles;
   const size_t esz = (f64 || i8) ? sizeof(double) : sizeof(float);
@@ -1311,7 +1300,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   if (nj) wb.Jpart = sizeof(double) * nj * nsj * nn;
   wb.Dp = sizeof(double) * std::max(nj, 1) * c->dstride;
   wb.gamma = sizeof(double) * std::max(nj, 1) * naux;
-  wb.gpart = sizeof(double) * naux * c->mtiles64;
+  wb.gpart = sizeof(double) * (f64 && fused ? nj * nopt::half_f64_gstride(naux, nbf) : (long)naux * c->mtiles64);
   wb.gslot = sizeof(double) * nopt::gamma_partial_blocks(c->nlslots, c->nlseg) * std::max(nj, 1) * naux;
   Work w;
   rc = work_area ? carve_work(work_area, work_area_bytes, wb, &w) : context_work(c, wb, &w);
@@ -1366,7 +1355,8 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     if (!overlap) mark(ph);
   };
   auto coulomb_gamma = [&]() -> hipError_t {
-    if (fused) {
+    if (fused && f64) {  // nothing: the J kernel adds the half-transform's partials
+    } else if (fused) {
       k_gamma<<<(naux + 255) / 256, 256, 0, sj>>>(w.gpart, c->mtiles, naux, w.gamma);
     } else if (i8 && rec) {
       nopt::ListRec r[2];
@@ -1405,7 +1395,9 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     const size_t jlds = sizeof(double) * nj * ((naux + nsj - 1) / nsj);  // at most JCHUNK_MAX values
 #define NOPT_JP(ND)                                                                                     \
   case ND:                                                                                              \
-    k_jpart<ND><<<gj, 256, jlds, sj>>>(c->B64, c->ld64, nbf, naux, w.gamma, naux, Jpart, (long)nsj * nn); \
+    k_jpart<ND><<<gj, 256, jlds, sj>>>(c->B64, c->ld64, nbf, naux, f64 && fused ? w.gpart : w.gamma,         \
+                                       f64 && fused ? nopt::half_f64_gstride(naux, nbf) : (long)naux,      \
+                                       f64 && fused ? nopt::kHalfF64Rows : 0, Jpart, (long)nsj * nn);      \
     break;
     switch (nj) { NOPT_JP(1) NOPT_JP(2) NOPT_JP(3) NOPT_JP(4) }
 #undef NOPT_JP
@@ -1501,11 +1493,11 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       }
     }
     else if (f64)
-      e = launch_half<double>(nt, gh, s, c->B64, ldb, nbf, (const double*)w.Cp, w.Dp, (double*)w.X, ldx,
-                              w.gpart, c->mtiles);
+      e = nopt::launch_half_f64(nt, ngroups, fused ? nj : 0, s, c->B64, ldb, naux, nbf, (const double*)w.Cp, w.Dp,
+                                c->dstride, (double*)w.X, ldx, w.gpart);
     else if (prec == NOPT_PREC_FP32)
-      e = launch_half<float>(nt, gh, s, c->B64, ldb, nbf, (const float*)w.Cp, w.Dp, (float*)w.X, ldx,
-                             w.gpart, c->mtiles);
+      e = launch_half_f32(nt, gh, s, c->B64, ldb, nbf, (const float*)w.Cp, w.Dp, (float*)w.X, ldx,
+                          w.gpart, c->mtiles);
     else
       e = nopt::launch_half_bf16(prec == NOPT_PREC_BF16X3 ? 2 : 3, nt, gh, s, c->B64, ldb, nbf,
                                  (const float*)w.Cp, w.Dp, (float*)w.X, ldx, w.gpart, c->mtiles);
@@ -1685,8 +1677,12 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || ncu <= 0)
       ncu = 256;
-    // FP64 exchange: four blocks per CU fit, one round of them
-    c->nsk = (int)std::max(1L, std::min(naux, 4L * ncu / c->ntiles8));
+    // FP64 exchange: four blocks per CU fit; a small system takes two, so that
+    // a block has more functions per partial tile and the J pass room beside
+    // it: builds of 192, 250, 298 functions 286, 467, 683 us with two against
+    // 300, 487, 692 us with four, of 490 functions 3.15 against 3.01 ms
+    c->nsk = (int)std::max(1L, std::min(naux, std::max(2L * ncu / c->ntiles8,
+                                                       std::min(4L * ncu / c->ntiles8, naux / 64))));
     const long slots = 2L * ncu / 8;  // per XCD
     int best = 8;
     double best_eff = 0.0;
@@ -1713,7 +1709,11 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
     return set_error(NOPT_EHIP, std::string("nopt_jk_create: ") + hip_msg(e));
   }
   const long nn = nbf * nbf;
-  if (!rc) rc = dev_alloc((void**)&c->gpart, sizeof(double) * naux * c->mtiles64, "gamma partials");
+  if (!rc)
+    rc = dev_alloc((void**)&c->gpart,
+                   sizeof(double) * std::max(naux * c->mtiles64,
+                                             nopt::kHalfF64Dens * nopt::half_f64_gstride(naux, nbf)),
+                   "gamma partials");
   if (!rc) rc = dev_alloc((void**)&c->gamma, sizeof(double) * kMaxBatch * naux, "gamma");
   if (!rc) {
     static_assert(nopt::kSyrkI8Tile == nopt::kSyrkF64Tile, "ntiles8 counts the tiles of both");
