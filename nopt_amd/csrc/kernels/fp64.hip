@@ -284,6 +284,111 @@ __global__ __launch_bounds__(256, 4) void k_syrk_f64(const double* __restrict__ 
         Kt[(wr + i * 16 + acc_row<double>(lane, v)) * T + wc + j * 16 + lr] = acc[i][j][v];
 }
 
+// ---------------------------------------------------- active-space integrals
+// R_Q[a2][a1] = sum_mn C2[a2][n] B_Q[m][n] C1[a1][m] for one Q per block (Cp:
+// the rows of C2, then those of C1, ldc values each, zero from nbf on).
+//
+// Bound by the read of B, of which only the lower triangle W (diagonal halved)
+// is read: R = C2 W^T C1^T + C2 W C1^T. A wave takes strips of 16 rows in
+// zigzag order (their lengths grow with the row), forms U = W [C2; C1]^T of the
+// strip on the matrix cores, and adds both products with the strip's columns of
+// C1 and C2: U leaves the accumulators in the layout of either operand (lane
+// l, item v: row l / 16 + 4 v, column l % 16), so it goes back into the matrix
+// unit as it is. The waves' sums are added in their order. R is written in
+// groups of 32 functions, [Q / 32][a2*na + a1][Q % 32] (zero for Q >= naux), the
+// form in which the exchange kernel contracts it over Q.
+// For 240 functions, 1160 auxiliary functions and 10 active orbitals 106 us
+// (958 us with one row at a time per wave on the vector unit, lane sums after
+// every row), and 5 us for the contraction over Q (290 us in one thread per
+// element).
+template <int NT>
+__global__ __launch_bounds__(256, NT == 1 ? 4 : 2) void k_active_half(const double* __restrict__ B, long ld, int nbf,
+                                                                      int naux, const double* __restrict__ Cp,
+                                                                      int ldc, int na, double* __restrict__ R) {
+  __shared__ double part[4][NT * NT * 256];
+  const int Q = blockIdx.x, t = threadIdx.x, lane = t & 63, lr = lane & 15, g = lane >> 4, w = t >> 6;
+  double* Rq = R + (long)(Q / kActiveGroup) * na * na * kActiveGroup + Q % kActiveGroup;
+  if (Q >= naux) {
+    for (int e = t; e < na * na; e += 256) Rq[(long)e * kActiveGroup] = 0.0;
+    return;
+  }
+  const double* Bq = B + (long)Q * nbf * ld + 2 * g;
+  // rows of C2 (tiles 0 .. NT-1) and C1 (NT .. 2 NT-1); rows beyond na repeat the last one (not written)
+  const double* cp[2 * NT];
+#pragma unroll
+  for (int j = 0; j < 2 * NT; ++j)
+    cp[j] = Cp + (long)((j < NT ? 0 : na) + min((j % NT) * 16 + lr, na - 1)) * ldc;
+  d4_t r[NT][NT];  // [a2 tile][a1 tile]
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) r[i][j] = d4_t{0, 0, 0, 0};
+  const int ns = (nbf + 15) / 16;
+  for (int rnd = 0; 4 * rnd < ns; ++rnd) {
+    const int st = 4 * rnd + ((rnd & 1) ? 3 - w : w), m0 = 16 * st;
+    if (st >= ns) continue;
+    const double* br = Bq + (long)min(m0 + lr, nbf - 1) * ld;
+    d4_t u[2 * NT];
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j) u[j] = d4_t{0, 0, 0, 0};
+    d2_t b[2], bn[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) b[h] = *reinterpret_cast<const d2_t*>(br + 8 * h);
+    for (int n0 = 0; n0 <= m0; n0 += 16) {
+      d2_t c[2 * NT][2];
+#pragma unroll
+      for (int j = 0; j < 2 * NT; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) c[j][h] = *reinterpret_cast<const d2_t*>(cp[j] + n0 + 8 * h + 2 * g);
+      const int nn = n0 < m0 ? n0 + 16 : n0;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) bn[h] = *reinterpret_cast<const d2_t*>(br + nn + 8 * h);
+      if (n0 == m0) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int n = 8 * h + 2 * g + e;
+            b[h][e] = n < lr ? b[h][e] : n == lr ? 0.5 * b[h][e] : 0.0;
+          }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int j = 0; j < 2 * NT; ++j) u[j] = mfma_f64(b[h][e], c[j][h][e], u[j]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) b[h] = bn[h];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      double cm[2 * NT];
+#pragma unroll
+      for (int j = 0; j < 2 * NT; ++j) cm[j] = cp[j][m0 + 4 * v + g];
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          r[i][j] = mfma_f64(u[i][v], cm[NT + j], r[i][j]);
+          r[i][j] = mfma_f64(cm[i], u[NT + j][v], r[i][j]);
+        }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        part[w][(i * 16 + acc_row<double>(lane, v)) * (16 * NT) + j * 16 + lr] = r[i][j][v];
+  __syncthreads();
+  for (int e = t; e < na * na; e += 256) {
+    const int i = (e / na) * (16 * NT) + e % na;
+    Rq[(long)e * kActiveGroup] = ((part[0][i] + part[1][i]) + part[2][i]) + part[3][i];
+  }
+}
+
 }  // namespace
 
 int half_f64_nt(long ncol, int* groups) {
@@ -317,6 +422,18 @@ hipError_t launch_half_f64(int nt, int groups, int nd, hipStream_t s, const doub
 #undef NOPT_HALF_F64_ND
 #undef NOPT_HALF_F64
   return nt < 1 || nt > 8 ? hipErrorInvalidValue : hipGetLastError();
+}
+
+hipError_t launch_active_half(hipStream_t s, const double* B, long ld, int nbf, int naux, const double* Cp, int ldc,
+                              int na, double* R) {
+  if (na < 1 || na > 32 || ldc < (nbf + 15) / 16 * 16 || ldc % 2 || ld < (nbf + 15) / 16 * 16)
+    return hipErrorInvalidValue;
+  const unsigned grid = (unsigned)((naux + kActiveGroup - 1) / kActiveGroup * kActiveGroup);
+  if (na <= 16)
+    k_active_half<1><<<grid, 256, 0, s>>>(B, ld, nbf, naux, Cp, ldc, na, R);
+  else
+    k_active_half<2><<<grid, 256, 0, s>>>(B, ld, nbf, naux, Cp, ldc, na, R);
+  return hipGetLastError();
 }
 
 int syrk_f64_splits(int nsplit, int naux, int kpad) {

@@ -21,6 +21,16 @@ int half_f64_nt(long ncol, int* groups);
 hipError_t launch_half_f64(int nt, int groups, int nd, hipStream_t s, const double* B, long ld, int naux, int nbf,
                            const double* Cp, const double* Dp, long dstride, double* X, long ldx, double* gpart);
 
+// R_Q[a2][a1] = sum_mn C2[a2][n] B_Q[m][n] C1[a1][m], na <= 32, B symmetric
+// (rows of ld values, zero from nbf to the next multiple of 16): Cp holds the
+// na rows of C2, then those of C1, ldc values each (ldc a multiple of 16, zero
+// from nbf on). R[Q / G][a2*na + a1][Q % G], G = kActiveGroup, zero for
+// Q >= naux: the X of launch_syrk_f64 with na*na rows, ldx = kpad = G and
+// ceil(naux / G) functions.
+constexpr int kActiveGroup = 32;
+hipError_t launch_active_half(hipStream_t s, const double* B, long ld, int nbf, int naux, const double* Cp, int ldc,
+                              int na, double* R);
+
 constexpr int kSyrkF64Tile = 64;  // exchange tile edge
 
 // Kpart[split][tile][r][c] = sum over the split's functions Q of

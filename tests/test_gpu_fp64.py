@@ -59,3 +59,22 @@ def test_fp64_build_at_tile_edges(nbf, naux, nocc):
         J2, K2 = ctx.build(D, C, prec="fp64")
         assert np.array_equal(J, J2) and np.array_equal(K, K2)
         assert np.array_equal(ctx.build(None, C, prec="fp64", J=False)[1], K)
+
+
+@pytest.mark.parametrize("nbf,naux,na", [(1, 1, 1), (16, 31, 4), (17, 33, 16), (63, 32, 17), (64, 5, 8), (130, 40, 32)])
+def test_active_integrals_at_tile_edges(nbf, naux, na):
+    """Two different orbital sets: ints = sum_Q R_Q R_Q, R_Q = C2 B_Q C1^T."""
+    say("nbf", nbf, "naux", naux, "na", na)
+    B, packed, _, _ = inputs(nbf, naux, 1)
+    rng = np.random.default_rng(4)
+    C1, C2 = rng.standard_normal((2, na, nbf))
+
+    def ints(B, C1, C2):
+        R = np.einsum("bn,qmn,am->qba", C2, B, C1, optimize=True).reshape(naux, na * na)
+        return R.T @ R
+
+    with JKContext(nbf, naux, keep="fp64") as ctx:
+        ctx.set_B_fitted(packed)
+        for _ in range(2):
+            got = ctx.active_ints(C1, C2).reshape(na * na, na * na)
+            check(got, ints(B, C1, C2), ints(np.abs(B), np.abs(C1), np.abs(C2)), 4 * nbf + naux + 2)
