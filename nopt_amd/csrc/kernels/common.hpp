@@ -56,6 +56,14 @@ __device__ __forceinline__ double warp_sum(double v) {
   return v;
 }
 
+// the value of x in lane l (l the same for the whole wave)
+__device__ __forceinline__ double lane_read(double x, int l) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+
 // block-wide sum over 256 threads; result valid in thread 0
 __device__ __forceinline__ double block_sum256(double v, double* sh /* >= 4 */) {
   v = warp_sum(v);

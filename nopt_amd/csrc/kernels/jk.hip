@@ -886,15 +886,15 @@ int find_live(nopt_jk_ctx* c) {
 
 // Forms B from packed lower-triangle rows in host memory, host[P][m(m+1)/2+n]:
 // raw (P|mn) solved against the Cholesky factor dL of the metric (B = L^-1
-// (P|mn)), or an already fitted tensor when dL is null. The rows m stream
-// through the device in chunks (whole rows, at most kChunkBytes), so the
-// packed tensor is never resident: each chunk is copied in, solved, and
-// written into the kept forms of B: FP64 rows, and the digit planes (split
+// (P|mn), dXd the inverses of its diagonal blocks), or an already fitted tensor
+// when dL is null. The rows m stream through the device in chunks (whole rows,
+// at most kChunkBytes), so the packed tensor is never resident: each chunk is
+// copied in, solved, and written into the kept forms of B: FP64 rows, and the digit planes (split
 // from the FP64 rows, or, without them, from the chunks in a second pass once
 // every row maximum is known).
 constexpr size_t kChunkBytes = (size_t)4 << 30;
 
-int form_B(nopt_jk_ctx* c, const double* host, const double* dL) {
+int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* dXd) {
   const bool keep64 = !(c->flags & NOPT_CTX_INT8_ONLY), keep8 = !(c->flags & NOPT_CTX_FP64_ONLY);
   const long na = c->naux, nbf = c->nbf, rows = na * nbf;
   const long cp = std::max(nbf, std::min(c->npair, (long)(kChunkBytes / (sizeof(double) * na))));
@@ -942,7 +942,7 @@ int form_B(nopt_jk_ctx* c, const double* host, const double* dL) {
         const long p0 = (long)m0 * (m0 + 1) / 2, w = (long)m1 * (m1 + 1) / 2 - p0;
         HIPCHK(hipMemcpy2DAsync(dA, sizeof(double) * w, host + p0, sizeof(double) * c->npair, sizeof(double) * w,
                                 na, hipMemcpyHostToDevice, s));
-        if (dL) HIPCHK(nopt::trsm_lower_f64(dL, na, (int)na, dA, w, w, s));
+        if (dL) HIPCHK(nopt::trsm_lower_f64(dL, na, (int)na, dXd, dA, w, w, s));
         if (keep64) {
           HIPCHK(nopt::unpack_packed_f64(dA, w, m0, m1, (int)nbf, na, c->B64, c->ld64, s));
         } else if (pass == 0) {
@@ -2051,11 +2051,11 @@ int nopt_jk_set_B(nopt_jk_ctx* c, const double* eri3, const double* metric) {
   rc = order_in(c, c->stream);
   if (rc) return rc;
   const long na = c->naux;
-  double* dV = nullptr;
-  rc = dev_alloc((void**)&dV, sizeof(double) * na * na, "metric");
+  double* dV = nullptr;  // the metric, then its factor; behind it the inverses of the factor's diagonal blocks
+  rc = dev_alloc((void**)&dV, sizeof(double) * (na * na + nopt::chol_inverse_count((int)na)), "metric");
   if (!rc) {
     hipError_t e = hipMemcpyAsync(dV, metric, sizeof(double) * na * na, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = nopt::cholesky_f64(dV, na, (int)na, c->info, c->stream);
+    if (e == hipSuccess) e = nopt::cholesky_f64(dV, na, (int)na, dV + na * na, c->info, c->stream);
     int info = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&info, c->info, sizeof(int), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -2064,7 +2064,7 @@ int nopt_jk_set_B(nopt_jk_ctx* c, const double* eri3, const double* metric) {
     else if (info != 0)
       rc = set_error(NOPT_ECHOL, "Coulomb metric is not positive definite (pivot " + std::to_string(info - 1) + ")");
   }
-  if (!rc) rc = form_B(c, eri3, dV);
+  if (!rc) rc = form_B(c, eri3, dV, dV + na * na);
   dev_free(dV);
   return rc;
 }
@@ -2076,7 +2076,7 @@ int nopt_jk_set_B_fitted(nopt_jk_ctx* c, const double* Bp) {
   if (!Bp) return set_error(NOPT_EINVAL, "nopt_jk_set_B_fitted: null input");
   rc = order_in(c, c->stream);
   if (rc) return rc;
-  return form_B(c, Bp, nullptr);
+  return form_B(c, Bp, nullptr, nullptr);
 }
 
 int nopt_jk_get_B(nopt_jk_ctx* c, double* Bp) {

@@ -950,12 +950,6 @@ __device__ __forceinline__ double row_ror(double x) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), 0x120 + N, 0xf, 0xf, false);
   return __builtin_bit_cast(double, (unsigned long long)(unsigned)lo | ((unsigned long long)(unsigned)hi << 32));
 }
-__device__ __forceinline__ double lane_read(double x, int l) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
-}
 __device__ __forceinline__ double wave_sum_rows(double v) {
   v += row_ror<8>(v);
   v += row_ror<4>(v);

@@ -78,3 +78,22 @@ def test_active_integrals_at_tile_edges(nbf, naux, na):
         for _ in range(2):
             got = ctx.active_ints(C1, C2).reshape(na * na, na * na)
             check(got, ints(B, C1, C2), ints(np.abs(B), np.abs(C1), np.abs(C2)), 4 * nbf + naux + 2)
+
+
+@pytest.mark.parametrize("naux,nbf", [(1, 1), (16, 3), (63, 16), (64, 15), (65, 17), (130, 24), (200, 9)])
+def test_fitted_tensor_at_block_edges(naux, nbf):
+    """B = L^-1 (P|mn) from a metric of condition about ten: the error of a
+    Cholesky factorisation and a substitution is below naux u cond(V) relative
+    to the columns' norms (a factor 8 for the constants of both)."""
+    say("naux", naux, "nbf", nbf)
+    rng = np.random.default_rng(6)
+    A = rng.standard_normal((naux, naux))
+    V = A @ A.T / naux + np.eye(naux)
+    T = rng.standard_normal((naux, nbf * (nbf + 1) // 2))
+    want = np.linalg.solve(np.linalg.cholesky(V), T)
+    with JKContext(nbf, naux, keep="fp64") as ctx:
+        ctx.set_B(T, V)
+        got = ctx.get_B()
+    tol = 8.0 * naux * 2.0 ** -53 * np.linalg.cond(V) * np.linalg.norm(T, axis=0)
+    say("  max error / bound", float(np.max(np.abs(got - want) / tol)))
+    assert np.all(np.abs(got - want) <= tol)
