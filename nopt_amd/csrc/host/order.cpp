@@ -1,8 +1,6 @@
 // Reverse Cuthill-McKee order of the basis functions (declared in order.hpp).
 #include "order.hpp"
 
-#include <omp.h>
-
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -41,25 +39,13 @@ Levels bfs(const std::vector<std::vector<int>>& adj, const std::vector<int>& deg
 
 }  // namespace
 
-void band_order(const double* T, long nrow, long nbf, int* perm) {
-  const long npair = nbf * (nbf + 1) / 2;
-  std::vector<double> mx((size_t)npair, 0.0);
-#pragma omp parallel
-  {
-    // each thread owns a contiguous range of pairs (m, n) over every row P
-    const int nt = omp_get_num_threads(), id = omp_get_thread_num();
-    const long a = npair * id / nt, b = npair * (id + 1) / nt;
-    for (long P = 0; P < nrow; ++P) {
-      const double* r = T + P * npair;
-      for (long k = a; k < b; ++k) mx[(size_t)k] = std::max(mx[(size_t)k], std::fabs(r[k]));
-    }
-  }
+void band_order(const double* mx, long nbf, int* perm) {
   std::vector<std::vector<int>> adj((size_t)nbf);
   for (long m = 0; m < nbf; ++m) {
-    const double dm = mx[(size_t)(m * (m + 1) / 2 + m)];
+    const double dm = mx[m * (m + 1) / 2 + m];
     for (long n = 0; n < m; ++n) {
-      const double dn = mx[(size_t)(n * (n + 1) / 2 + n)];
-      if (mx[(size_t)(m * (m + 1) / 2 + n)] > std::ldexp(std::sqrt(dm * dn), -30)) {
+      const double dn = mx[n * (n + 1) / 2 + n];
+      if (mx[m * (m + 1) / 2 + n] > std::ldexp(std::sqrt(dm * dn), -30)) {
         adj[(size_t)m].push_back((int)n);
         adj[(size_t)n].push_back((int)m);
       }

@@ -31,6 +31,7 @@
 
 #include "../../../include/nopt_jk.h"
 #include "../host/errors.hpp"
+#include "../host/hostcopy.hpp"
 #include "../host/order.hpp"
 #include "common.hpp"
 #include "bf16.hpp"
@@ -614,6 +615,10 @@ struct nopt_jk_ctx {
   double *dJ = nullptr, *dK = nullptr, *dD = nullptr, *dC = nullptr, *dH = nullptr,
          *dF = nullptr, *dG = nullptr, *epart = nullptr, *dE = nullptr;
   long dC_cap = 0;
+  // pinned pieces of large host-to-device copies (upload_rows) and the events of their last use
+  void* ring[2] = {};
+  hipEvent_t ring_ev[2] = {};
+  unsigned ring_pos = 0;
   double* act = nullptr;  // workspace of the active integrals
   size_t act_bytes = 0;
   double *xD[kMaxBatch - 1] = {}, *xC[kMaxBatch - 1] = {}, *xJ[kMaxBatch - 1] = {}, *xK[kMaxBatch - 1] = {};
@@ -724,6 +729,15 @@ template <typename P>
 void dev_free(P*& p) {
   if (p) (void)hipFree((void*)p);
   p = nullptr;
+}
+
+void free_ring(nopt_jk_ctx* c) {
+  for (int b = 0; b < 2; ++b) {
+    if (c->ring[b]) (void)hipHostFree(c->ring[b]);
+    if (c->ring_ev[b]) (void)hipEventDestroy(c->ring_ev[b]);
+    c->ring[b] = nullptr;
+    c->ring_ev[b] = nullptr;
+  }
 }
 
 // Grows a device buffer to at least `bytes`.
@@ -884,55 +898,130 @@ int find_live(nopt_jk_ctx* c) {
   return rc;
 }
 
+// Host to device: rows of `width` bytes at `pitch` in host memory to contiguous
+// rows at dst, on stream s. A copy from pageable memory runs at 19 (strided) to
+// 29 GB/s in one host thread, so larger transfers pass through two pinned
+// pieces, filled by several threads while the other one is on its way (about
+// 50 GB/s); the context keeps the pieces. Without them (small transfers, no
+// pinned memory to be had) the runtime's own copy.
+constexpr size_t kRingBytes = (size_t)8 << 20, kRingMin = (size_t)32 << 20;
+int upload_rows(nopt_jk_ctx* c, char* dst, const char* src, size_t width, size_t pitch, long rows, hipStream_t s) {
+  if (!c->ring[0]) {
+    HIPCHK(hipMemcpy2DAsync(dst, width, src, pitch, width, rows, hipMemcpyHostToDevice, s));
+    return NOPT_OK;
+  }
+  const long rpp = std::max(1L, (long)(kRingBytes / width));  // rows per piece; a longer row in parts
+  for (long r = 0; r < rows; r += rpp) {
+    const long nr = std::min(rpp, rows - r);
+    for (size_t o = 0; o < width; o += kRingBytes) {
+      const size_t w = std::min(width - o, kRingBytes);
+      const int b = c->ring_pos++ & 1;
+      HIPCHK(hipEventSynchronize(c->ring_ev[b]));
+      nopt::copy_rows((char*)c->ring[b], src + (size_t)r * pitch + o, w, pitch, nr);
+      HIPCHK(hipMemcpyAsync(dst + (size_t)r * width + o, c->ring[b], w * (size_t)nr, hipMemcpyHostToDevice, s));
+      HIPCHK(hipEventRecord(c->ring_ev[b], s));
+    }
+  }
+  return NOPT_OK;
+}
+
 // Forms B from packed lower-triangle rows in host memory, host[P][m(m+1)/2+n]:
 // raw (P|mn) solved against the Cholesky factor dL of the metric (B = L^-1
 // (P|mn), dXd the inverses of its diagonal blocks), or an already fitted tensor
 // when dL is null. The rows m stream through the device in chunks (whole rows,
 // at most kChunkBytes), so the packed tensor is never resident: each chunk is
-// copied in, solved, and written into the kept forms of B: FP64 rows, and the digit planes (split
-// from the FP64 rows, or, without them, from the chunks in a second pass once
-// every row maximum is known).
-constexpr size_t kChunkBytes = (size_t)4 << 30;
+// copied in, solved, and written into the kept forms of B: FP64 rows, and the
+// digit planes (split from the FP64 rows, or, without them, from the chunks in
+// a second pass once every row maximum is known). A chunk's auxiliary functions
+// arrive on the side stream in groups of whole 64-row blocks, and each group is
+// solved while the next one is on its way. The weights of the band order are
+// the maxima over P of the chunks as they arrive. info: the factorisation's
+// status on its way to the host on c->stream, looked at before any form of B is
+// touched.
+constexpr size_t kChunkBytes = (size_t)4 << 30, kGroupBytes = (size_t)16 << 20;
 
-int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* dXd) {
+int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* dXd, const int* info) {
   const bool keep64 = !(c->flags & NOPT_CTX_INT8_ONLY), keep8 = !(c->flags & NOPT_CTX_FP64_ONLY);
   const long na = c->naux, nbf = c->nbf, rows = na * nbf;
   const long cp = std::max(nbf, std::min(c->npair, (long)(kChunkBytes / (sizeof(double) * na))));
   int rc = NOPT_OK;
-  c->b_ready = false;
-  if (keep64 && !c->B64) rc = dev_alloc((void**)&c->B64, sizeof(double) * rows * c->ld64, "B (FP64)");
-  if (!rc && keep8 && !c->Be) {
-    if (c->bfull) rc = dev_alloc((void**)&c->Bd, (size_t)4 * rows * c->ld8, "B digit planes");
-    if (!rc) rc = dev_alloc((void**)&c->Be, sizeof(int) * rows, "B row exponents");
-    if (!rc) rc = dev_alloc((void**)&c->Be8, (size_t)na * c->ld8, "B row exponents (bytes)");
-    c->splane = na * 16L * c->nseg;
-    if (!rc) rc = dev_alloc((void**)&c->Bs, (size_t)5 * c->splane, "packed lower triangle of B");
-    c->nmb = (int)((nbf + 31) / 32);
-    if (!rc && c->ld8 <= 2048) rc = dev_alloc((void**)&c->Bm, sizeof(uint32_t) * na * c->nmb, "slab masks of B");
-    if (!rc) rc = dev_alloc((void**)&c->perm, sizeof(int) * nbf, "order of the functions");
-    if (!rc) rc = dev_alloc((void**)&c->pinv, sizeof(int) * nbf, "inverse order of the functions");
-  }
-  if (rc) return rc;
-  if (keep8) {
-    std::vector<int> hp((size_t)nbf), hi((size_t)nbf);
-    nopt::band_order(host, na, nbf, hp.data());
-    for (long i = 0; i < nbf; ++i) hi[(size_t)hp[(size_t)i]] = (int)i;
-    if (hipMemcpy(c->perm, hp.data(), sizeof(int) * nbf, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->pinv, hi.data(), sizeof(int) * nbf, hipMemcpyHostToDevice) != hipSuccess)
-      return set_error(NOPT_EHIP, "form_B: copy of the function order failed");
-  }
-  double* dA = nullptr;
+  double *dA = nullptr, *mx = nullptr;
   unsigned long long* rmax = nullptr;
   rc = dev_alloc((void**)&dA, sizeof(double) * na * cp, "chunk of the packed tensor");
+  if (!rc && keep8) rc = dev_alloc((void**)&mx, sizeof(double) * c->npair, "pair maxima");
   if (!rc && keep8 && !keep64) rc = dev_alloc((void**)&rmax, sizeof(unsigned long long) * rows, "row maxima");
-  auto run = [&]() -> int {
-    hipStream_t s = c->stream;
+  if (!rc && !c->ring[0] && sizeof(double) * na * c->npair >= kRingMin) {
+    bool ok = true;
+    for (int b = 0; b < 2 && ok; ++b)
+      ok = hipHostMalloc(&c->ring[b], kRingBytes, hipHostMallocDefault) == hipSuccess &&
+           hipEventCreateWithFlags(&c->ring_ev[b], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      free_ring(c);
+    }
+  }
+  hipStream_t s = c->stream, up = c->side;
+  hipEvent_t ev = nullptr;
+  // the functions' order from the pair maxima, once all chunks have been seen
+  auto set_order = [&]() -> int {
+    std::vector<double> h((size_t)c->npair);
+    std::vector<int> hp((size_t)nbf), hi((size_t)nbf);
+    HIPCHK(hipMemcpyAsync(h.data(), mx, sizeof(double) * c->npair, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    nopt::band_order(h.data(), nbf, hp.data());
+    for (long i = 0; i < nbf; ++i) hi[(size_t)hp[(size_t)i]] = (int)i;
+    HIPCHK(hipMemcpyAsync(c->perm, hp.data(), sizeof(int) * nbf, hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(c->pinv, hi.data(), sizeof(int) * nbf, hipMemcpyHostToDevice, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return NOPT_OK;
+  };
+  // copies the pairs p0 .. p0 + w of every function into dA and solves them
+  auto load_chunk = [&](long p0, long w, bool maxima) -> int {
+    const long per = std::max(1L, (long)(kGroupBytes / (64 * sizeof(double) * w))) * 64;
+    HIPCHK(hipEventRecord(ev, s));  // dA is free again
+    HIPCHK(hipStreamWaitEvent(up, ev, 0));
+    for (long r0 = 0; r0 < na; r0 += per) {
+      const long r1 = std::min(na, r0 + per);
+      const int r = upload_rows(c, (char*)(dA + r0 * w), (const char*)(host + r0 * c->npair + p0), sizeof(double) * w,
+                                sizeof(double) * c->npair, r1 - r0, up);
+      if (r) return r;
+      HIPCHK(hipEventRecord(ev, up));
+      HIPCHK(hipStreamWaitEvent(s, ev, 0));
+      if (maxima) HIPCHK(nopt::pair_max(dA + r0 * w, w, r1 - r0, mx + p0, s));
+      if (dL) HIPCHK(nopt::trsm_lower_f64(dL, na, (int)na, dXd, dA, w, w, (int)r0, (int)r1, s));
+    }
+    return NOPT_OK;
+  };
+  // buffers of the kept forms, and their padding cleared
+  auto prepare_forms = [&]() -> int {
+    int r = NOPT_OK;
+    c->b_ready = false;
+    if (keep64 && !c->B64) r = dev_alloc((void**)&c->B64, sizeof(double) * rows * c->ld64, "B (FP64)");
+    if (!r && keep8 && !c->Be) {
+      if (c->bfull) r = dev_alloc((void**)&c->Bd, (size_t)4 * rows * c->ld8, "B digit planes");
+      if (!r) r = dev_alloc((void**)&c->Be, sizeof(int) * rows, "B row exponents");
+      if (!r) r = dev_alloc((void**)&c->Be8, (size_t)na * c->ld8, "B row exponents (bytes)");
+      c->splane = na * 16L * c->nseg;
+      if (!r) r = dev_alloc((void**)&c->Bs, (size_t)5 * c->splane, "packed lower triangle of B");
+      c->nmb = (int)((nbf + 31) / 32);
+      if (!r && c->ld8 <= 2048) r = dev_alloc((void**)&c->Bm, sizeof(uint32_t) * na * c->nmb, "slab masks of B");
+      if (!r) r = dev_alloc((void**)&c->perm, sizeof(int) * nbf, "order of the functions");
+      if (!r) r = dev_alloc((void**)&c->pinv, sizeof(int) * nbf, "inverse order of the functions");
+    }
+    if (r) return r;
     if (keep64) HIPCHK(hipMemsetAsync(c->B64, 0, sizeof(double) * rows * c->ld64, s));
     if (rmax) {
       if (c->Bd) HIPCHK(hipMemsetAsync(c->Bd, 0, (size_t)4 * rows * c->ld8, s));
       HIPCHK(hipMemsetAsync(c->Bs, 0, (size_t)5 * c->splane, s));  // the scatter leaves the padding
       HIPCHK(hipMemsetAsync(rmax, 0, sizeof(unsigned long long) * rows, s));
     }
+    return NOPT_OK;
+  };
+  auto run = [&]() -> int {
+    HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    if (mx) HIPCHK(hipMemsetAsync(mx, 0, sizeof(double) * c->npair, s));
+    bool ready = false;
+    int r;
     // pass 1 forms the FP64 rows or the row maxima, pass 2 (integer forms
     // without FP64 rows) the packed triangle and the digit planes
     for (int pass = 0; pass < (rmax ? 2 : 1); ++pass) {
@@ -940,13 +1029,20 @@ int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* d
         int m1 = m0 + 1;
         while (m1 < (int)nbf && (long)(m1 + 1) * (m1 + 2) / 2 - (long)m0 * (m0 + 1) / 2 <= cp) ++m1;
         const long p0 = (long)m0 * (m0 + 1) / 2, w = (long)m1 * (m1 + 1) / 2 - p0;
-        HIPCHK(hipMemcpy2DAsync(dA, sizeof(double) * w, host + p0, sizeof(double) * c->npair, sizeof(double) * w,
-                                na, hipMemcpyHostToDevice, s));
-        if (dL) HIPCHK(nopt::trsm_lower_f64(dL, na, (int)na, dXd, dA, w, w, s));
+        // (a single chunk is still there in the second pass)
+        if ((pass == 0 || w < c->npair) && (r = load_chunk(p0, w, keep8 && pass == 0))) return r;
+        if (!ready) {
+          HIPCHK(hipStreamSynchronize(s));
+          if (info && *info)
+            return set_error(NOPT_ECHOL,
+                             "Coulomb metric is not positive definite (pivot " + std::to_string(*info - 1) + ")");
+          if ((r = prepare_forms())) return r;
+          ready = true;
+        }
         if (keep64) {
           HIPCHK(nopt::unpack_packed_f64(dA, w, m0, m1, (int)nbf, na, c->B64, c->ld64, s));
         } else if (pass == 0) {
-          HIPCHK(nopt::rowmax_packed(dA, w, m0, m1, (int)nbf, na, rmax, s, c->pinv));
+          HIPCHK(nopt::rowmax_packed(dA, w, m0, m1, (int)nbf, na, rmax, s));
         } else {
           HIPCHK(nopt::scatter_segs_chunk(dA, w, m0, m1, (int)nbf, na, c->Be, c->pinv, c->nseg, c->Bs, c->splane, s));
           if (c->Bd)
@@ -955,7 +1051,8 @@ int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* d
         }
         m0 = m1;
       }
-      if (rmax && pass == 0) HIPCHK(nopt::rowmax_exponents(rmax, rows, c->Be, s));
+      if (pass == 0 && keep8 && (r = set_order())) return r;
+      if (rmax && pass == 0) HIPCHK(nopt::rowmax_exponents(rmax, rows, c->Be, s, c->pinv, (int)nbf));
     }
     if (keep64 && keep8) {
       // the exponents (and digit planes) from the FP64 rows, then the packed triangle
@@ -969,7 +1066,13 @@ int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* d
     return NOPT_OK;
   };
   if (!rc) rc = run();
+  if (rc) {  // copies and kernels may still be under way
+    (void)hipStreamSynchronize(up);
+    (void)hipStreamSynchronize(s);
+  }
+  if (ev) (void)hipEventDestroy(ev);
   dev_free(dA);
+  dev_free(mx);
   dev_free(rmax);
   if (!rc && keep8) rc = find_live(c);
   if (!rc) c->b_ready = true;
@@ -1736,6 +1839,7 @@ void nopt_jk_destroy(nopt_jk_ctx* c) {
   dev_free(c->epart);
   dev_free(c->dE);
   dev_free(c->act);
+  free_ring(c);
   dev_free(c->info);
   dev_free(c->Bd);
   dev_free(c->Be);
@@ -2056,15 +2160,16 @@ int nopt_jk_set_B(nopt_jk_ctx* c, const double* eri3, const double* metric) {
   if (!rc) {
     hipError_t e = hipMemcpyAsync(dV, metric, sizeof(double) * na * na, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = nopt::cholesky_f64(dV, na, (int)na, dV + na * na, c->info, c->stream);
-    int info = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&info, c->info, sizeof(int), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    int* info = nullptr;  // pinned, so that its copy does not hold up the host
+    if (e == hipSuccess) e = hipHostMalloc((void**)&info, sizeof(int), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMemcpyAsync(info, c->info, sizeof(int), hipMemcpyDeviceToHost, c->stream);
     if (e != hipSuccess)
       rc = set_error(NOPT_EHIP, std::string("metric factorisation: ") + hip_msg(e));
-    else if (info != 0)
-      rc = set_error(NOPT_ECHOL, "Coulomb metric is not positive definite (pivot " + std::to_string(info - 1) + ")");
+    else
+      rc = form_B(c, eri3, dV, dV + na * na, info);
+    (void)hipStreamSynchronize(c->stream);
+    if (info) (void)hipHostFree(info);
   }
-  if (!rc) rc = form_B(c, eri3, dV, dV + na * na);
   dev_free(dV);
   return rc;
 }
@@ -2076,7 +2181,7 @@ int nopt_jk_set_B_fitted(nopt_jk_ctx* c, const double* Bp) {
   if (!Bp) return set_error(NOPT_EINVAL, "nopt_jk_set_B_fitted: null input");
   rc = order_in(c, c->stream);
   if (rc) return rc;
-  return form_B(c, Bp, nullptr, nullptr);
+  return form_B(c, Bp, nullptr, nullptr, nullptr);
 }
 
 int nopt_jk_get_B(nopt_jk_ctx* c, double* Bp) {

@@ -320,8 +320,8 @@ __global__ __launch_bounds__(512) void k_panel(double* A, long lda, int n, int k
   }
 }
 
-// B (n x ncol, ldb) <- L^-1 B, 128 columns per block from the first to the last
-// row block without leaving the kernel: for each block of 64 rows the products
+// B (n x ncol, ldb) <- L^-1 B for the rows r0 .. r1, 128 columns per block from
+// the first to the last row block without leaving the kernel: for each block of 64 rows the products
 // of L with the rows solved so far (slabs of 16 terms of both through
 // double-buffered LDS, as in k_gemm_f64; the solved rows come back from the
 // block's own stores), then the diagonal block. Eight waves of 32 x 32.
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(512) void k_panel(double* A, long lda, int n, int k
 // over all rows below, took 6.4 and 58 ms.
 __global__ __launch_bounds__(512, 4) void k_trsm_f64(const double* __restrict__ L, long ldl, int n,
                                                      const double* __restrict__ Xd, double* B, long ldb,
-                                                     long ncol) {
+                                                     long ncol, int r0, int r1) {
   __shared__ __attribute__((aligned(16))) double sm[NB * kTS];
   double(*As)[64][18] = reinterpret_cast<double(*)[64][18]>(sm);                   // [2]
   double(*Bs)[16][kTS] = reinterpret_cast<double(*)[16][kTS]>(sm + 2 * 64 * 18);   // [2]
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(512, 4) void k_trsm_f64(const double* __restrict__ 
   // loader: L value (row t / 16 + 32 u, term t % 16), B value (term t / 128 + 4 u, column t % 128)
   const int ar = t >> 4, ak = t & 15, bk = t >> 7, bn = t & 127;
   const double* pb = B + min(c0 + bn, ncol - 1);
-  for (int k0 = 0; k0 < n; k0 += NB) {
+  for (int k0 = r0; k0 < r1; k0 += NB) {
     const int kb = min(NB, n - k0);
     d4_t acc[2][2], tt[2][2];
 #pragma unroll
@@ -459,11 +459,11 @@ hipError_t cholesky_f64(double* A, long lda, int n, double* Xd, int* d_info, hip
   return hipGetLastError();
 }
 
-hipError_t trsm_lower_f64(const double* L, long ldl, int n, const double* Xd, double* B, long ldb, long ncol,
-                          hipStream_t s) {
-  if (ncol <= 0) return hipSuccess;
-  if (ncol > 128L * 0x7fffffff) return hipErrorInvalidValue;
-  k_trsm_f64<<<(unsigned)((ncol + 127) / 128), 512, 0, s>>>(L, ldl, n, Xd, B, ldb, ncol);
+hipError_t trsm_lower_f64(const double* L, long ldl, int n, const double* Xd, double* B, long ldb, long ncol, int r0,
+                          int r1, hipStream_t s) {
+  if (ncol <= 0 || r0 >= r1) return hipSuccess;
+  if (ncol > 128L * 0x7fffffff || r0 < 0 || r0 % NB || r1 > n || (r1 < n && r1 % NB)) return hipErrorInvalidValue;
+  k_trsm_f64<<<(unsigned)((ncol + 127) / 128), 512, 0, s>>>(L, ldl, n, Xd, B, ldb, ncol, r0, r1);
   return hipGetLastError();
 }
 

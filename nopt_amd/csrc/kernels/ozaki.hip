@@ -221,9 +221,27 @@ __global__ __launch_bounds__(256) void k_packed_tiles(const double* __restrict__
   }
 }
 
-__global__ void k_rowmax_exponent(const unsigned long long* __restrict__ rowmax, long rows, int* __restrict__ expo) {
+__global__ void k_rowmax_exponent(const unsigned long long* __restrict__ rowmax, long rows, int* __restrict__ expo,
+                                  const int* __restrict__ pinv, int nbf) {
   const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < rows) expo[r] = row_exponent(__longlong_as_double((long long)rowmax[r]));
+  if (r >= rows) return;
+  expo[pinv ? r / nbf * nbf + pinv[r % nbf] : r] = row_exponent(__longlong_as_double((long long)rowmax[r]));
+}
+
+// mx[p] = max(mx[p], max_r |A[r*w + p]|): a pair per thread, eight rows in flight
+__global__ __launch_bounds__(256) void k_pair_max(const double* __restrict__ A, long w, long rows,
+                                                  double* __restrict__ mx) {
+  const long p = (long)blockIdx.x * 256 + threadIdx.x;
+  if (p >= w) return;
+  double m = mx[p];
+  for (long r = 0; r < rows; r += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = A[(r + u < rows ? r + u : rows - 1) * w + p];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) m = fmax(m, fabs(v[u]));
+  }
+  mx[p] = m;
 }
 
 // ------------------------------------------------ packed lower triangle of B
@@ -1467,8 +1485,14 @@ hipError_t rowmax_packed(const double* A, long cp, int m0, int m1, int nbf, long
   return hipGetLastError();
 }
 
-hipError_t rowmax_exponents(const unsigned long long* rowmax, long rows, int* expo, hipStream_t s) {
-  if (rows > 0) k_rowmax_exponent<<<(unsigned)((rows + 255) / 256), 256, 0, s>>>(rowmax, rows, expo);
+hipError_t rowmax_exponents(const unsigned long long* rowmax, long rows, int* expo, hipStream_t s, const int* pinv,
+                            int nbf) {
+  if (rows > 0) k_rowmax_exponent<<<(unsigned)((rows + 255) / 256), 256, 0, s>>>(rowmax, rows, expo, pinv, nbf);
+  return hipGetLastError();
+}
+
+hipError_t pair_max(const double* A, long w, long rows, double* mx, hipStream_t s) {
+  if (w > 0 && rows > 0) k_pair_max<<<(unsigned)((w + 255) / 256), 256, 0, s>>>(A, w, rows, mx);
   return hipGetLastError();
 }
 

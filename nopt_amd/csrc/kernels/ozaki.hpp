@@ -27,7 +27,11 @@ hipError_t unpack_packed_f64(const double* A, long cp, int m0, int m1, int nbf, 
                              hipStream_t s);
 hipError_t rowmax_packed(const double* A, long cp, int m0, int m1, int nbf, long naux, unsigned long long* rowmax,
                          hipStream_t s, const int* pinv = nullptr);
-hipError_t rowmax_exponents(const unsigned long long* rowmax, long rows, int* expo, hipStream_t s);
+// (with pinv: row m of each function to row pinv[m] of expo, nbf rows a function)
+hipError_t rowmax_exponents(const unsigned long long* rowmax, long rows, int* expo, hipStream_t s,
+                            const int* pinv = nullptr, int nbf = 1);
+// mx[p] = max(mx[p], max over the rows of |A[r*w + p]|), p < w (NaNs left out)
+hipError_t pair_max(const double* A, long w, long rows, double* mx, hipStream_t s);
 hipError_t split_packed_i8(const double* A, long cp, int m0, int m1, int nbf, long naux, const int* expo, int ns,
                            int8_t* planes, long ldo, long pstride, hipStream_t s, const int* pinv = nullptr);
 // Digit split of the half-transformed rows fused into the half-transform:
