@@ -11,7 +11,7 @@ namespace nopt {
 void copy_rows(char* dst, const char* src, size_t width, size_t pitch, long rows) {
   const size_t total = width * (size_t)rows;
   if (!total) return;
-  const int nt = (int)std::min<size_t>((size_t)std::min(8, omp_get_max_threads()), (total >> 18) + 1);
+  const int nt = (int)std::min<size_t>((size_t)std::min(4, omp_get_max_threads()), (total >> 18) + 1);
 #pragma omp parallel num_threads(nt)
   {
     // each thread a contiguous range of dst

@@ -901,9 +901,11 @@ int find_live(nopt_jk_ctx* c) {
 // Host to device: rows of `width` bytes at `pitch` in host memory to contiguous
 // rows at dst, on stream s. A copy from pageable memory runs at 19 (strided) to
 // 29 GB/s in one host thread, so larger transfers pass through two pinned
-// pieces, filled by several threads while the other one is on its way (about
-// 50 GB/s); the context keeps the pieces. Without them (small transfers, no
-// pinned memory to be had) the runtime's own copy.
+// pieces, one filled by several threads while the other is on its way; the
+// context keeps the pieces. One copy at a time: with the next one queued behind
+// it the pair ran at 28 GB/s, so at 37. 303 MB take 8.3 ms (pieces of 16 MB
+// 7.9), 16.5 as one strided copy. Without the pieces (small transfers, no pinned
+// memory to be had) the runtime's own copy.
 constexpr size_t kRingBytes = (size_t)8 << 20, kRingMin = (size_t)32 << 20;
 int upload_rows(nopt_jk_ctx* c, char* dst, const char* src, size_t width, size_t pitch, long rows, hipStream_t s) {
   if (!c->ring[0]) {
@@ -918,6 +920,7 @@ int upload_rows(nopt_jk_ctx* c, char* dst, const char* src, size_t width, size_t
       const int b = c->ring_pos++ & 1;
       HIPCHK(hipEventSynchronize(c->ring_ev[b]));
       nopt::copy_rows((char*)c->ring[b], src + (size_t)r * pitch + o, w, pitch, nr);
+      HIPCHK(hipEventSynchronize(c->ring_ev[b ^ 1]));  // one copy at a time
       HIPCHK(hipMemcpyAsync(dst + (size_t)r * width + o, c->ring[b], w * (size_t)nr, hipMemcpyHostToDevice, s));
       HIPCHK(hipEventRecord(c->ring_ev[b], s));
     }
