@@ -86,6 +86,18 @@ __device__ __forceinline__ void tri_tile(int t, int& bi, int& bj) {
 
 static inline long round_up(long x, long m) { return (x + m - 1) / m * m; }
 
+// element e of dst[r][c] (ldd) = src[r'][c'] (lds) for r < rows, c < cols, zero
+// elsewhere in [0, rows_pad) x [0, ldd); r' = rperm[r], c' = cperm[c] (each optional)
+template <typename T>
+__device__ __forceinline__ void pad_copy(long e, const double* __restrict__ src, long lds, int rows, int cols,
+                                         T* __restrict__ dst, long ldd, int rows_pad, const int* __restrict__ rperm,
+                                         const int* __restrict__ cperm) {
+  if (e >= (long)rows_pad * ldd) return;
+  const long r = e / ldd, c = e % ldd;
+  const double v = (r < rows && c < cols) ? src[(rperm ? rperm[r] : r) * lds + (cperm ? cperm[c] : c)] : 0.0;
+  dst[e] = (T)v;
+}
+
 // Work lists: one launch runs a kernel over the grids of several items (the
 // systems of a ragged batch). Item i owns the blocks [first[i], first[i+1])
 // of the 1-D launch; a kernel body sees its block of the item's own grid as

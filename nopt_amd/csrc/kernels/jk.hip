@@ -61,23 +61,11 @@ __global__ void k_pack_B(const double* __restrict__ B64, long ld64, int nbf, lon
   Bp[e] = B64[(Q * nbf + a) * ld64 + b];
 }
 
-// dst[r][c] (ldd) = src[r'][c'] (lds) for r < rows, c < cols; zero elsewhere
-// in [0, rows_pad) x [0, ldd); r' = rperm[r], c' = cperm[c] (each optional)
-template <typename T>
-__device__ __forceinline__ void k_pad_copy_body(const VB vb, const double* __restrict__ src, long lds, int rows,
-                                                int cols, T* __restrict__ dst, long ldd, int rows_pad,
-                                                const int* __restrict__ rperm, const int* __restrict__ cperm) {
-  const long e = (long)vb.x * blockDim.x + threadIdx.x;
-  if (e >= (long)rows_pad * ldd) return;
-  const long r = e / ldd, c = e % ldd;
-  double v = (r < rows && c < cols) ? src[(rperm ? rperm[r] : r) * lds + (cperm ? cperm[c] : c)] : 0.0;
-  dst[e] = (T)v;
-}
 template <typename T>
 __global__ void k_pad_copy(const double* __restrict__ src, long lds, int rows, int cols,
                            T* __restrict__ dst, long ldd, int rows_pad, const int* __restrict__ rperm,
                            const int* __restrict__ cperm) {
-  k_pad_copy_body<T>(grid_vb(), src, lds, rows, cols, dst, ldd, rows_pad, rperm, cperm);
+  pad_copy<T>((long)blockIdx.x * blockDim.x + threadIdx.x, src, lds, rows, cols, dst, ldd, rows_pad, rperm, cperm);
 }
 // work-list form (FP64 copies)
 struct ItemPad {
@@ -95,8 +83,8 @@ struct ItemPad {
 __global__ void k_pad_copy_list(const ItemPad* __restrict__ items, const int* __restrict__ first, int n) {
   const int i = list_item(first, n, (int)blockIdx.x);
   const ItemPad& a = items[i];
-  k_pad_copy_body<double>(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz), a.src, a.lds, a.rows, a.cols, a.dst,
-                          a.ldd, a.rows_pad, a.rperm, a.cperm);
+  pad_copy<double>((long)((int)blockIdx.x - first[i]) * blockDim.x + threadIdx.x, a.src, a.lds, a.rows, a.cols, a.dst,
+                   a.ldd, a.rows_pad, a.rperm, a.cperm);
 }
 
 // ---------------------------------------------------- half-transform (FP32)
@@ -691,6 +679,9 @@ struct nopt_jk_ctx {
 };
 
 namespace {
+// largest triangle of B (in FP64, times the densities) of which a build runs in
+// line on one stream
+constexpr size_t kInlineBytes = (size_t)64 << 20;
 constexpr int kPhases = 6;  // staging, half-transform, gamma, J partials, exchange, J output
 constexpr int kTimedBuilds = 512;
 }  // namespace
@@ -1349,7 +1340,6 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   Work w;
   rc = work_area ? carve_work(work_area, work_area_bytes, wb, &w) : context_work(c, wb, &w);
   if (rc) return rc;
-  double* Jpart = (double*)w.Jpart;
   const bool tm = !rec && c->timing && c->timed < kTimedBuilds;
   auto mark = [&](int ph) {
     if (tm) (void)hipEventRecord(c->tev[(size_t)c->timed * (kPhases + 1) + ph], s);
@@ -1358,7 +1348,15 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   // run on the side stream, forked after the staging (after the
   // half-transform in the integer mode, or when gamma rides on it) and joined
   // before the build ends, so that they overlap the exchange.
-  const bool overlap = !rec && !tm && nj > 0 && anyK;
+  // A small build runs in line instead: its Coulomb pair is over sooner than
+  // the second stream has taken it up and been waited for (two hops of about
+  // 10 us), and J and K of a density leave in one launch. Water clusters, one
+  // density, microseconds in line and with the second stream: 24 functions 26
+  // and 63 (FP64), 31 and 52 (int8), 96 functions 46 and 59, 55 and 70, 144
+  // functions 93 and 97, 87 and 100, 192 functions 174 and 168, 153 and 159;
+  // two densities cross at about half that size.
+  const bool inl = !rec && !tm && sizeof(double) * (double)naux * (double)c->npair * std::max(nj, 1) <= (double)kInlineBytes;
+  const bool overlap = !rec && !tm && nj > 0 && anyK && !inl;
   const dim3 gfin((unsigned)((nbf + kFinCols - 1) / kFinCols), (unsigned)nbf);  // output blocks
   // the integer mode works on the functions in the order of B's integer
   // forms (perm[new] = old): densities are read through it, orbitals'
@@ -1376,15 +1374,13 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   };
   auto split_rows = [&](const double* src, long ld, int cols, long rows_src, int8_t* planes, long ldo, long rows_dst,
                         long pstride, int* expo, const int* cperm = nullptr) -> hipError_t {
-    if (!rec)
-      return nopt::split_rows_i8(src, ld, cols, rows_src, 4, planes, ldo, rows_dst, pstride, expo, s, nullptr, 0,
-                                 cperm);
     if (rows_dst <= 0) return hipSuccess;
     nopt::ListRec r;
     CHK_(nopt::split_rows_item(src, ld, cols, rows_src, 4, planes, ldo, rows_dst, pstride, expo, &r, cperm));
     rec->add(1, r);
     return hipSuccess;
   };
+  double* Jpart = (double*)w.Jpart;
   auto finalize = [&](int phase, const double* Jp, int nsj_, const double* Kp, int nsk_, int ntl, int kt,
                       double* J, double* K, hipStream_t st) {
     const uint8_t* jl = Jp && i8 ? c->jlive : nullptr;  // J partials of the integer pair
@@ -1411,7 +1407,9 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       return hipSuccess;
     } else if (i8) {
       CHK_(nopt::launch_gamma_slots(nj, c->nsg, sj, c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lslots,
-                                    c->nlslots, c->lsegs, c->nlseg, w.Dp, ldb, c->dstride, w.gslot, w.gamma, naux));
+                                    c->nlslots, c->lsegs, c->nlseg, w.Dp, ldb, c->dstride, w.gslot,
+                                    nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj) ? nullptr : w.gamma,
+                                    naux));
     } else {
 #define NOPT_GF(ND)                                                                                         \
   case ND:                                                                                                  \
@@ -1432,9 +1430,12 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       rec->add(5, r);
       return hipSuccess;
     }
-    if (i8)
+    if (i8) {
+      const int nsb = nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj);
       return nopt::launch_jpart_slots(nj, nsj, sj, c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lslots,
-                                      c->nlslots, c->lsegs, c->nlseg, w.gamma, naux, Jpart, (long)nsj * nn);
+                                      c->nlslots, c->lsegs, c->nlseg, nsb ? w.gslot : w.gamma, naux, nsb, Jpart,
+                                      (long)nsj * nn);
+    }
     dim3 gj((nbf + 1) / 2, nsj);
     const size_t jlds = sizeof(double) * nj * ((naux + nsj - 1) / nsj);  // at most JCHUNK_MAX values
 #define NOPT_JP(ND)                                                                                     \
@@ -1451,9 +1452,10 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     CHK_(coulomb_gamma());
     return coulomb_j();
   };
+  bool jout[kMaxBatch] = {};  // J already written
   auto coulomb_out = [&]() -> hipError_t {
     for (int k = 0; k < nj; ++k)
-      finalize(6, Jpart + (long)k * nsj * nn, nsj, nullptr, 0, 1, KT, it[jl[k]].J, nullptr, sj);
+      if (!jout[k]) finalize(6, Jpart + (long)k * nsj * nn, nsj, nullptr, 0, 1, KT, it[jl[k]].J, nullptr, sj);
     return hipGetLastError();
   };
   // 0: no J; 1: forked after staging; 2: in line (after the half-transform)
@@ -1461,8 +1463,23 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   mark(0);
   // densities of the J list into slots 0..nj-1 (ld = ldb); orbital blocks
   // into the stacked factor at column offsets off[d] (zero rows between)
-  for (int k = 0; k < nj; ++k) pad_rows(0, it[jl[k]].D, nbf, nbf, nbf, w.Dp + k * c->dstride, ldb, nbf, perm, perm);
-  if (anyK) {
+  if (!rec && (f64 || i8)) {  // all of it in one launch
+    nopt::StageList sl;
+    for (int k = 0; k < nj; ++k)
+      sl.copy(it[jl[k]].D, nbf, nbf, nbf, w.Dp + k * c->dstride, ldb, nbf, perm, perm);
+    auto factor = [&](const double* src, int r, long o, int pad) {
+      if (i8)
+        sl.digits(src, nbf, nbf, r, (int8_t*)w.Cd + o * c->ld8, c->ld8, pad, ldx * c->ld8, (int*)w.Ce + o, perm);
+      else
+        sl.copy(src, nbf, r, nbf, (double*)w.Cp + o * ldb, ldb, pad);
+    };
+    for (int d = 0; d < nd && anyK; ++d) factor(it[d].C, (int)it[d].nocc, off[d], (int)(off[d + 1] - off[d]));
+    if (anyK) factor(nullptr, 0, ncol, (int)(ldx - ncol));
+    HIPCHK(nopt::launch_stage(sl, s));
+  } else {
+    for (int k = 0; k < nj; ++k) pad_rows(0, it[jl[k]].D, nbf, nbf, nbf, w.Dp + k * c->dstride, ldb, nbf, perm, perm);
+  }
+  if (anyK && (rec || !(f64 || i8))) {
     for (int d = 0; d < nd; ++d) {
       const int pad = (int)(off[d + 1] - off[d]);
       if (!pad) continue;
@@ -1470,8 +1487,6 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       if (i8)
         HIPCHK(split_rows(it[d].C, nbf, nbf, r, (int8_t*)w.Cd + off[d] * c->ld8, c->ld8, pad, ldx * c->ld8,
                           (int*)w.Ce + off[d], perm));
-      else if (f64)
-        stage_rows<double>(it[d].C, nbf, r, nbf, (double*)w.Cp + off[d] * ldb, ldb, pad, s);
       else
         stage_rows<float>(it[d].C, nbf, r, nbf, (float*)w.Cp + off[d] * ldb, ldb, pad, s);
     }
@@ -1479,8 +1494,6 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     if (i8)
       HIPCHK(split_rows(w.Dp, ldb, 0, 0, (int8_t*)w.Cd + ncol * c->ld8, c->ld8, tail, ldx * c->ld8,
                         (int*)w.Ce + ncol));
-    else if (f64)
-      stage_rows<double>(w.Dp, ldb, 0, 0, (double*)w.Cp + ncol * ldb, ldb, tail, s);
     else
       stage_rows<float>(w.Dp, ldb, 0, 0, (float*)w.Cp + ncol * ldb, ldb, tail, s);
   }
@@ -1561,6 +1574,15 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   }
   if (coulomb_at == 2) HIPCHK(coulomb());
   mark(4);
+  // K of density d, in line together with its J
+  auto out_k = [&](int d, const double* Kp, int nsk_, int ntl, int kt) {
+    int k = 0;
+    while (k < nj && jl[k] != d) ++k;
+    const bool both = inl && coulomb_at == 2 && k < nj;
+    if (both) jout[k] = true;
+    finalize(8, both ? Jpart + (long)k * nsj * nn : nullptr, nsj, Kp, nsk_, ntl, kt, both ? it[d].J : nullptr, it[d].K,
+             s);
+  };
   for (int d = 0; d < nd; ++d) {
     if (!it[d].K) continue;
     const int kpad = (int)(off[d + 1] - off[d]);
@@ -1598,8 +1620,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
         HIPCHK(nopt::launch_syrk_i8(c->ntiles8, c->nsk8, s, (const int8_t*)w.Xd, rows * ldk, (const int*)w.Xe, ldk,
                                     nbf, (int)naux, w.Kpart));
       }
-      finalize(8, nullptr, 0, w.Kpart + kfirst * kseg, nsum * c->nsk8, c->ntiles8, nopt::kSyrkI8Tile, nullptr,
-               it[d].K, s);
+      out_k(d, w.Kpart + kfirst * kseg, nsum * c->nsk8, c->ntiles8, nopt::kSyrkI8Tile);
     } else {
       const int ns = f64 ? nopt::syrk_f64_splits(c->nsk, naux, kpad) : c->nsk128();
       const int ntl = f64 ? c->ntiles8 : c->ntiles;
@@ -1611,7 +1632,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       else
         HIPCHK(nopt::launch_syrk_bf16(prec == NOPT_PREC_BF16X3 ? 2 : 3, gk, s, (const float*)w.X + off[d], ldx,
                                       nbf, naux, kpad, w.Kpart));
-      finalize(8, nullptr, 0, w.Kpart, ns, ntl, f64 ? nopt::kSyrkF64Tile : KT, nullptr, it[d].K, s);
+      out_k(d, w.Kpart, ns, ntl, f64 ? nopt::kSyrkF64Tile : KT);
     }
     HIPCHK(hipGetLastError());
   }

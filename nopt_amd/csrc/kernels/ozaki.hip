@@ -84,13 +84,12 @@ __host__ __device__ __forceinline__ long seg0(int m) {
 // padded) and row exponents. One wavefront per row. Optional reorders:
 // output row r reads source row (r/rper)*rper + rperm[r%rper], output column
 // c source column cperm[c].
-__device__ __forceinline__ void k_split_rows_body(const VB vb, const double* __restrict__ src, long ld, int cols,
+__device__ __forceinline__ void k_split_rows_body(const long row, const int lane, const double* __restrict__ src,
+                                                   long ld, int cols,
                                                    long rows_src, int ns, int8_t* __restrict__ planes,
                                                    long ldo, long pstride, int* __restrict__ expo,
                                                    const int* __restrict__ rperm, long rper,
                                                    const int* __restrict__ cperm) {
-  const long row = vb.x;
-  const int lane = threadIdx.x;
   const bool live = row < rows_src;
   const double* s = src + (rperm ? row / rper * rper + rperm[row % rper] : row) * ld;
   double mx = 0.0;
@@ -113,16 +112,33 @@ __global__ __launch_bounds__(64) void k_split_rows(const double* __restrict__ sr
                                                    long ldo, long pstride, int* __restrict__ expo,
                                                    const int* __restrict__ rperm, long rper,
                                                    const int* __restrict__ cperm) {
-  k_split_rows_body(grid_vb(), src, ld, cols, rows_src, ns, planes, ldo, pstride, expo, rperm, rper, cperm);
+  k_split_rows_body(blockIdx.x, threadIdx.x, src, ld, cols, rows_src, ns, planes, ldo, pstride, expo, rperm, rper, cperm);
 }
 __global__ __launch_bounds__(64) void k_split_rows_list(const ItemSplit* __restrict__ items,
     const int* __restrict__ first, int n) {
   const int i = list_item(first, n, (int)blockIdx.x);
   const ItemSplit& a = items[i];
-  k_split_rows_body(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz),
+  k_split_rows_body((int)blockIdx.x - first[i], threadIdx.x,
       a.src, a.ld, a.cols, a.rows_src, a.ns, a.planes, a.ldo, a.pstride, a.expo, nullptr, 0, a.cperm);
 }
 
+// The staging of a build: block b finds its item, a copy (256 elements) or a
+// digit split (four rows, one per wave).
+__global__ __launch_bounds__(256) void k_stage(StageList l) {
+  int i = l.n - 1;
+  while (i > 0 && l.it[i].first > (int)blockIdx.x) --i;
+  const StageItem& a = l.it[i];
+  const int b = (int)blockIdx.x - a.first;
+  if (!a.expo) {
+    pad_copy<double>((long)b * 256 + threadIdx.x, a.src, a.lds, a.rows, a.cols, (double*)a.dst, a.ldd, a.rows_pad,
+                     a.rperm, a.cperm);
+  } else {
+    const long row = 4L * b + (threadIdx.x >> 6);
+    if (row < a.rows_pad)
+      k_split_rows_body(row, threadIdx.x & 63, a.src, a.lds, a.cols, a.rows, 4, (int8_t*)a.dst, a.ldd, a.pstride,
+                        a.expo, nullptr, 0, a.cperm);
+  }
+}
 
 // ------------------------------------------- rows of packed symmetric chunks
 // A chunk of a symmetric tensor in packed lower-triangle form,
@@ -1126,8 +1142,12 @@ __global__ __launch_bounds__(256) void k_gamma_sum_list(const ItemGammaSum* __re
 // each thread owns SPL slots (8 columns each) and accumulates over the Q of
 // its split in registers, loading the digits of the next Q while the current
 // one is accumulated.
+// With nsb > 0 gamma holds the partials of k_gamma_slots (nsb slot blocks),
+// which every block adds for the functions of its split, in the order of
+// k_gamma_sum, into gs (ND x the split's functions): a small system then has
+// one launch less.
 template <int ND, int SPL, bool SEG>
-__device__ __forceinline__ void k_jpart_slots_body(const VB vb, const int8_t* __restrict__ Bs, long splane, long sq,
+__device__ __forceinline__ void k_jpart_slots_body(const VB vb, double* gs, int nsb, const int8_t* __restrict__ Bs, long splane, long sq,
                                                      const int* __restrict__ Be, int nbf, int naux,
                                                      const int* __restrict__ slots, int nslots,
                                                      const double* __restrict__ gamma, long gstride,
@@ -1167,11 +1187,30 @@ __device__ __forceinline__ void k_jpart_slots_body(const VB vb, const int8_t* __
     }
   };
   if (q0 < q1) fetch(q0, cur, ecur);
+  const int len = q1 - q0;
+  if (nsb > 0) {
+    for (int e = threadIdx.x; e < ND * len; e += 256) {
+      const int d = e / len, q = q0 + e % len;
+      const double* g = gamma + (long)d * naux + q;
+      const long st = (long)ND * naux;
+      double s[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int b = 0; b < nsb; b += 4) {
+        double v[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[p] = g[(long)min(b + p, nsb - 1) * st];
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (b + p < nsb) s[p] += v[p];
+      }
+      gs[e] = ((s[0] + s[1]) + s[2]) + s[3];
+    }
+    __syncthreads();
+  }
   for (int q = q0; q < q1; ++q) {
     if (q + 1 < q1) fetch(q + 1, nxt, enxt);
     double g[ND];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) g[d] = gamma[d * gstride + q];
+    for (int d = 0; d < ND; ++d) g[d] = nsb > 0 ? gs[d * len + q - q0] : gamma[d * gstride + q];
 #pragma unroll
     for (int k = 0; k < SPL; ++k) {
       double bv[8];
@@ -1206,9 +1245,10 @@ template <int ND, int SPL, bool SEG>
 __global__ __launch_bounds__(256) void k_jpart_slots(const int8_t* __restrict__ Bs, long splane, long sq,
                                                      const int* __restrict__ Be, int nbf, int naux,
                                                      const int* __restrict__ slots, int nslots,
-                                                     const double* __restrict__ gamma, long gstride,
+                                                     const double* __restrict__ gamma, long gstride, int nsb,
                                                      double* __restrict__ Jpart, long jstride) {
-  k_jpart_slots_body<ND, SPL, SEG>(grid_vb(),
+  extern __shared__ double gs[];
+  k_jpart_slots_body<ND, SPL, SEG>(grid_vb(), gs, nsb,
       Bs, splane, sq, Be, nbf, naux, slots, nslots, gamma, gstride, Jpart, jstride);
 }
 template <int ND, int SPL, bool SEG>
@@ -1216,7 +1256,7 @@ __global__ __launch_bounds__(256) void k_jpart_slots_list(const ItemJ* __restric
     const int* __restrict__ first, int n) {
   const int i = list_item(first, n, (int)blockIdx.x);
   const ItemJ& a = items[i];
-  k_jpart_slots_body<ND, SPL, SEG>(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz),
+  k_jpart_slots_body<ND, SPL, SEG>(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz), nullptr, 0,
       a.Bs, a.splane, a.sq, a.Be, a.nbf, a.naux, a.slots, a.nslots, a.gamma, a.gstride, a.Jpart, a.jstride);
 }
 
@@ -1461,6 +1501,20 @@ hipError_t split_rows_i8(const double* src, long ld, int cols, long rows_src, in
   return hipGetLastError();
 }
 
+hipError_t launch_stage(StageList& l, hipStream_t s) {
+  long b = 0;
+  for (int i = 0; i < l.n; ++i) {
+    StageItem& a = l.it[i];
+    if (a.rows > a.rows_pad || a.cols > a.ldd || (a.expo && a.pstride < (long)a.rows_pad * a.ldd))
+      return hipErrorInvalidValue;
+    a.first = (int)b;
+    b += a.expo ? (a.rows_pad + 3) / 4 : ((long)a.rows_pad * a.ldd + 255) / 256;
+  }
+  if (b > 0x7fffffffL) return hipErrorInvalidValue;
+  if (b > 0) k_stage<<<(unsigned)b, 256, 0, s>>>(l);
+  return hipGetLastError();
+}
+
 namespace {
 bool packed_chunk_ok(long cp, int m0, int m1, int nbf, long naux) {
   return m0 >= 0 && m1 <= nbf && m0 < m1 && naux > 0 && naux <= 65535 &&
@@ -1676,20 +1730,30 @@ hipError_t launch_gamma_slots(int nd, int nsplit, hipStream_t s, const int8_t* B
     case 4: k_gamma_slots<4, kGammaSPL, false><<<grid, 256, 0, s>>>(Bs, splane, sq, Be, nbf, naux, slots, nslots, Dp, ldd, dstride, gpart); break;
     default: return hipErrorInvalidValue;
   }
-  k_gamma_sum<<<dim3((naux + 63) / 64, nd), 256, 0, s>>>(gpart, (int)grid.x, nd, naux, gamma, gstride);
+  if (gamma)
+    k_gamma_sum<<<dim3((naux + 63) / 64, nd), 256, 0, s>>>(gpart, (int)grid.x, nd, naux, gamma, gstride);
   return hipGetLastError();
+}
+
+int gamma_slots_unsummed(int nd, int nslots, int nseg, int naux, int nsplit_j) {
+  // every J block adds the partials of its split's functions: worth a launch
+  // for few slot blocks (up to about 170 functions) and splits that fit LDS
+  const int nsb = nd <= 2 ? (nseg + 63) / 64 : gamma_slot_blocks(nslots);
+  return nsb <= 16 && (long)nd * ((naux + nsplit_j - 1) / nsplit_j) <= 4096 ? nsb : 0;
 }
 
 int gamma_partial_blocks(int nslots, int nseg) { return std::max(gamma_slot_blocks(nslots), (nseg + 63) / 64); }
 
 hipError_t launch_jpart_slots(int nd, int nsplit, hipStream_t s, const int8_t* Bs, long splane, long sq, const int* Be,
                               int nbf, int naux, const int* slots, int nslots, const int* segs, int nseg,
-                              const double* gamma, long gstride, double* Jpart, long jstride) {
+                              const double* gamma, long gstride, int nsb, double* Jpart, long jstride) {
+  const size_t lds = nsb > 0 ? sizeof(double) * nd * ((naux + nsplit - 1) / nsplit) : 0;
+  if (lds > 65536) return hipErrorInvalidValue;
   switch (nd) {
-    case 1: k_jpart_slots<1, 2, true><<<dim3((nseg + 255) / 256, nsplit), 256, 0, s>>>(Bs, splane, sq, Be, nbf, naux, segs, nseg, gamma, gstride, Jpart, jstride); break;
-    case 2: k_jpart_slots<2, 2, true><<<dim3((nseg + 255) / 256, nsplit), 256, 0, s>>>(Bs, splane, sq, Be, nbf, naux, segs, nseg, gamma, gstride, Jpart, jstride); break;
-    case 3: k_jpart_slots<3, 1, false><<<dim3((nslots + 255) / 256, nsplit), 256, 0, s>>>(Bs, splane, sq, Be, nbf, naux, slots, nslots, gamma, gstride, Jpart, jstride); break;
-    case 4: k_jpart_slots<4, 1, false><<<dim3((nslots + 255) / 256, nsplit), 256, 0, s>>>(Bs, splane, sq, Be, nbf, naux, slots, nslots, gamma, gstride, Jpart, jstride); break;
+    case 1: k_jpart_slots<1, 2, true><<<dim3((nseg + 255) / 256, nsplit), 256, lds, s>>>(Bs, splane, sq, Be, nbf, naux, segs, nseg, gamma, gstride, nsb, Jpart, jstride); break;
+    case 2: k_jpart_slots<2, 2, true><<<dim3((nseg + 255) / 256, nsplit), 256, lds, s>>>(Bs, splane, sq, Be, nbf, naux, segs, nseg, gamma, gstride, nsb, Jpart, jstride); break;
+    case 3: k_jpart_slots<3, 1, false><<<dim3((nslots + 255) / 256, nsplit), 256, lds, s>>>(Bs, splane, sq, Be, nbf, naux, slots, nslots, gamma, gstride, nsb, Jpart, jstride); break;
+    case 4: k_jpart_slots<4, 1, false><<<dim3((nslots + 255) / 256, nsplit), 256, lds, s>>>(Bs, splane, sq, Be, nbf, naux, slots, nslots, gamma, gstride, nsb, Jpart, jstride); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -13,6 +13,33 @@ namespace nopt {
 hipError_t split_rows_i8(const double* src, long ld, int cols, long rows_src, int ns, int8_t* planes, long ldo,
                          long rows_dst, long pstride, int* expo, hipStream_t s, const int* rperm = nullptr,
                          long rper = 0, const int* cperm = nullptr);
+// The staging of a build in one launch: zero-padded FP64 copies
+// (dst[r][c] = src[rperm[r]][cperm[c]], rows_pad rows of ldd) and digit splits
+// of orbital rows (split_rows_i8 with four planes).
+struct StageItem {
+  const double* src;
+  void* dst;
+  const int *rperm, *cperm;
+  int* expo;
+  long lds, ldd, pstride;
+  int rows, cols, rows_pad, first;  // first: the item's first block
+};
+struct StageList {
+  int n = 0;
+  StageItem it[9];
+  void add(const StageItem& x) {
+    if (x.rows_pad > 0) it[n++] = x;
+  }
+  void copy(const double* src, long lds, int rows, int cols, double* dst, long ldd, int rows_pad,
+            const int* rperm = nullptr, const int* cperm = nullptr) {
+    add({src, dst, rperm, cperm, nullptr, lds, ldd, 0, rows, cols, rows_pad, 0});
+  }
+  void digits(const double* src, long ld, int cols, int rows, int8_t* planes, long ldo, int rows_dst, long pstride,
+              int* expo, const int* cperm) {
+    add({src, planes, nullptr, cperm, expo, ld, ldo, pstride, rows, cols, rows_dst, 0});
+  }
+};
+hipError_t launch_stage(StageList& l, hipStream_t s);
 // Full rows from a chunk of a symmetric tensor kept as packed lower
 // triangles, A[P*cp + m(m+1)/2 + n - m0(m0+1)/2] for the rows m0 <= m < m1
 // (n <= m) of every P < naux: each element goes to both full rows it belongs
@@ -125,9 +152,13 @@ hipError_t launch_gamma_slots(int nd, int nsplit, hipStream_t s, const int8_t* B
                               int nbf, int naux, const int* slots, int nslots, const int* segs, int nseg,
                               const double* Dp, long ldd, long dstride, double* gpart, double* gamma, long gstride);
 int gamma_partial_blocks(int nslots, int nseg);
+// With a null gamma launch_gamma_slots leaves the sum of the partials to
+// launch_jpart_slots, which then gets gpart as its gamma and the number of slot
+// blocks as nsb: when gamma_slots_unsummed gives that number, not 0.
+int gamma_slots_unsummed(int nd, int nslots, int nseg, int naux, int nsplit_j);
 hipError_t launch_jpart_slots(int nd, int nsplit, hipStream_t s, const int8_t* Bs, long splane, long sq, const int* Be,
                               int nbf, int naux, const int* slots, int nslots, const int* segs, int nseg,
-                              const double* gamma, long gstride, double* Jpart, long jstride);
+                              const double* gamma, long gstride, int nsb, double* Jpart, long jstride);
 
 // Exchange partials over 64x64 lower-triangle tiles: Kpart[split][tile] for
 // ntiles tiles and nsplit Q-splits (each XCD a contiguous range of the
