@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -607,6 +608,7 @@ struct nopt_jk_ctx {
   void* ring[2] = {};
   hipEvent_t ring_ev[2] = {};
   unsigned ring_pos = 0;
+  bool ring_slow = false;  // filling the pieces is slow now (the rest of this tensor)
   double* act = nullptr;  // workspace of the active integrals
   size_t act_bytes = 0;
   double *xD[kMaxBatch - 1] = {}, *xC[kMaxBatch - 1] = {}, *xJ[kMaxBatch - 1] = {}, *xK[kMaxBatch - 1] = {};
@@ -896,21 +898,30 @@ int find_live(nopt_jk_ctx* c) {
 // context keeps the pieces. One copy at a time: with the next one queued behind
 // it the pair ran at 28 GB/s, so at 37. 303 MB take 8.3 ms (pieces of 16 MB
 // 7.9), 16.5 as one strided copy. Without the pieces (small transfers, no pinned
-// memory to be had) the runtime's own copy.
+// memory to be had) the runtime's own copy; and for the rest of a tensor once a
+// piece took kRingSlow seconds to fill (usually 0.15 ms): the process then has
+// more running threads than processors (a BLAS library's, still spinning after a
+// product), each of the copying threads can lose a time slice of some ms, and one
+// thread fares better: 589 MB right after a NumPy product took 98 ms, so 33 to 45
+// (22 with the processors free, 52 to 59 without pieces).
 constexpr size_t kRingBytes = (size_t)8 << 20, kRingMin = (size_t)32 << 20;
+constexpr double kRingSlow = 1e-3;
 int upload_rows(nopt_jk_ctx* c, char* dst, const char* src, size_t width, size_t pitch, long rows, hipStream_t s) {
-  if (!c->ring[0]) {
-    HIPCHK(hipMemcpy2DAsync(dst, width, src, pitch, width, rows, hipMemcpyHostToDevice, s));
-    return NOPT_OK;
-  }
   const long rpp = std::max(1L, (long)(kRingBytes / width));  // rows per piece; a longer row in parts
   for (long r = 0; r < rows; r += rpp) {
+    if (!c->ring[0] || c->ring_slow) {
+      HIPCHK(hipMemcpy2DAsync(dst + (size_t)r * width, width, src + (size_t)r * pitch, pitch, width, rows - r,
+                              hipMemcpyHostToDevice, s));
+      return NOPT_OK;
+    }
     const long nr = std::min(rpp, rows - r);
     for (size_t o = 0; o < width; o += kRingBytes) {
       const size_t w = std::min(width - o, kRingBytes);
       const int b = c->ring_pos++ & 1;
       HIPCHK(hipEventSynchronize(c->ring_ev[b]));
+      const auto t0 = std::chrono::steady_clock::now();
       nopt::copy_rows((char*)c->ring[b], src + (size_t)r * pitch + o, w, pitch, nr);
+      c->ring_slow |= std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > kRingSlow;
       HIPCHK(hipEventSynchronize(c->ring_ev[b ^ 1]));  // one copy at a time
       HIPCHK(hipMemcpyAsync(dst + (size_t)r * width + o, c->ring[b], w * (size_t)nr, hipMemcpyHostToDevice, s));
       HIPCHK(hipEventRecord(c->ring_ev[b], s));
@@ -944,6 +955,7 @@ int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* d
   rc = dev_alloc((void**)&dA, sizeof(double) * na * cp, "chunk of the packed tensor");
   if (!rc && keep8) rc = dev_alloc((void**)&mx, sizeof(double) * c->npair, "pair maxima");
   if (!rc && keep8 && !keep64) rc = dev_alloc((void**)&rmax, sizeof(unsigned long long) * rows, "row maxima");
+  c->ring_slow = false;
   if (!rc && !c->ring[0] && sizeof(double) * na * c->npair >= kRingMin) {
     bool ok = true;
     for (int b = 0; b < 2 && ok; ++b)
