@@ -408,6 +408,14 @@ __device__ __forceinline__ int row_max16(int x) {
   return max(x, ror16<1>(x));
 }
 
+// Waits for this wave's loads into LDS (a barrier then shows them to the block).
+__device__ __forceinline__ void lds_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// 16 bytes per lane from memory (vo: the lane's offset, so: the wave's) into the 1 KB of LDS at dst (the same for
+// the wave), lane after lane.
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, int8_t* dst, int vo, int so) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, 0);
+}
+
 // ------------------------------------------------------------ half-transform
 // LDS position of 16-byte chunk c (of a 64-byte k-slab) in row r: an XOR
 // swizzle under which the operand reads (ds_read_b128, lane l: row l % 16 of
@@ -457,8 +465,10 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
   constexpr int ACQ = 16 * BMI;                       // 16-byte B chunks per Q (4 planes x BMI rows x 4)
   constexpr int APT = ACQ * QPB / NTH;                // per thread
   constexpr int CCH = 4 * BN * 4;                     // 16-byte C chunks per slab
-  constexpr int CPT = (CCH + NTH - 1) / NTH;
-  static_assert(ACQ * QPB % NTH == 0 && NTH % (4 * BMI) == 0, "B slab must split evenly over the block");
+  constexpr int CPT = CCH / NTH;                      // per thread
+  static_assert(CCH % NTH == 0, "C slab must split evenly over the block");
+  static_assert(ACQ * QPB % NTH == 0 && NTH % (4 * BMI) == 0 && 4 * BMI % 64 == 0,
+                "B slab must split evenly over the block, a wave's part within a plane");
   __shared__ __attribute__((aligned(16))) int8_t sm[2][SB];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int qq = w / NW, w8 = w % NW;  // which Q of the block, wave within it
@@ -467,18 +477,24 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
   const long Qb = (long)vb.y * QPB;  // first Q of the block
   const long Q = Qb + qq;                  // this wave's Q
   const int cg = vb.z;
-  // B loader: chunk e = t + NTH u is chunk e%4 of row (e/4)%BMI in plane
-  // (e%ACQ)/(4 BMI) of the block's Q number e/ACQ (rows beyond nbf and a Q
-  // beyond naux load zeros); the row and chunk do not depend on u
-  const int ar = (t >> 2) % BMI, ac = t & 3;
-  const int8_t* ap[APT];
-  bool aok[APT];
+  // The operand slabs go from memory straight into LDS (no registers in between,
+  // so the next slab's loads are all under way while this one is multiplied): a
+  // wave's load fills 1 KB, lane l its 16-byte chunk l, and the swizzle is in
+  // which chunk of its row the lane asks for. B: LDS chunk e = t + NTH u holds
+  // row (e / 4) % BMI of plane (e % ACQ) / (4 BMI) of the block's Q number
+  // e / ACQ; function and plane are the same for a whole wave. Rows beyond nbf
+  // read row nbf - 1 and a Q beyond naux reads naux - 1 (both are masked below).
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  const int ar = (t >> 2) % BMI;
+  const int avo = (int)((min(m0 + ar, nbf - 1) - m0) * ld8) + 16 * swz(ar, t & 3);
+  __amdgpu_buffer_rsrc_t rA[PK ? 1 : APT];
   if constexpr (!PK) {
 #pragma unroll
     for (int u = 0; u < APT; ++u) {
-      const int e = t + NTH * u, qe = e / ACQ, pe = (e % ACQ) / (4 * BMI);
-      aok[u] = m0 + ar < nbf && Qb + qe < naux;
-      ap[u] = Bd + ((Qb + qe) * nbf + m0 + ar) * ld8 + 16 * ac + pe * bplane;
+      const int e = 64 * wu + NTH * u, qe = e / ACQ, pe = (e % ACQ) / (4 * BMI);
+      rA[u] = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<int8_t*>(Bd + pe * bplane + (min(Qb + qe, naux - 1L) * nbf + m0) * ld8), (short)0,
+          (int)(min(BMI, nbf - m0) * ld8), 0x00020000);
     }
   }
   // packed loader: GPT groups of four columns per thread and slab. Row-walk
@@ -489,7 +505,6 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
   constexpr int GPT = QPB * BMI * 16 / NTH;
   static_assert(!PK || (GPT * NTH == QPB * BMI * 16 && QPB * BMI == 64 && NWT * GPT == 16), "packed loader shape");
   const int tq = lane / BMI, tr = lane % BMI;  // column-walk: function and tile row of the lane
-  const int wu = __builtin_amdgcn_readfirstlane(w);
   // buffer resources from the block's first function (int32 byte offsets;
   // the ranges end with the last function, so loads beyond read zeros): the
   // N28 values, and the exponent bytes
@@ -514,23 +529,15 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
   uint4 praw[PK ? GPT : 1];   // N28 of the group's four columns
   uint32_t pexp[PK ? GPT : 1];  // column-walk: exponent bytes of the four stored rows
   int pn0 = 0, ptype = 0;       // slab of the prefetched values and its walk (0 rows, 1 columns, 2 diagonal block)
-  const int8_t* Cbase = Cd + (long)cg * BN * ld8;
-  // C loader: chunk e = t + NTH u < CCH of the slab is chunk (e & 3) of column
-  // (e >> 2) % BN in plane e / (4 BN); global and LDS offsets per u
-  int c_g[CPT], c_s[CPT];
+  // C: LDS chunk e = t + NTH u is in column (e / 4) % BN of plane e / (4 BN)
+  const __amdgpu_buffer_rsrc_t rC = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t*>(Cd + (long)cg * BN * ld8), (short)0, (int)(3 * cplane + BN * ld8), 0x00020000);
+  int cvo[CPT];
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
-    const int e = min(t + NTH * u, CCH - 1);
-    const int c = e & 3, col = (e >> 2) % BN, p = e / (4 * BN);
-    c_g[u] = (int)(p * cplane + (long)col * ld8 + 16 * c);
-    c_s[u] = QPB * AB + (p * BN + col) * KS + 16 * swz(col, c);
+    const int e = t + NTH * u, col = (e >> 2) % BN;
+    cvo[u] = (int)(e / (4 * BN) * cplane + col * ld8) + 16 * swz(col, t & 3);
   }
-  constexpr bool c_even = CCH % NTH == 0;
-  const bool c_last = c_even || t + NTH * (CPT - 1) < CCH;  // this thread has a chunk in the last round
-  // prefetch registers; the C chunks sit in two arrays of at most 16 dwords
-  // indexed with compile-time constants, so that both stay in registers
-  constexpr int CH = (CPT + 1) / 2;
-  uint4 a_reg[APT], c_lo[CH], c_hi[CPT - CH > 0 ? CPT - CH : 1];
 
   // packed slab at columns n0..n0+63: raw N28 (and exponent bytes) into registers
   auto gload_packed = [&](int n0) __attribute__((always_inline)) {
@@ -619,41 +626,14 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
       for (int p = 0; p < 4; ++p) *reinterpret_cast<uint32_t*>(base + p * BMI * KS) = pl[p];
     }
   };
-#define NOPT_GLOAD_A(k0)                                                                                 \
-  do {                                                                                                   \
-    if constexpr (PK) gload_packed(k0);                                                                  \
-    else                                                                                                 \
-      _Pragma("unroll") for (int u = 0; u < APT; ++u) a_reg[u] =                                         \
-          aok[u] ? *reinterpret_cast<const uint4*>(ap[u] + (k0)) : uint4{0, 0, 0, 0};                     \
-  } while (0)
-#define NOPT_GLOAD_C(k0)                                                                                 \
-  do {                                                                                                   \
-    static_for<CPT>([&](auto U) {                                                                        \
-      constexpr int u_ = decltype(U)::value;                                                             \
-      const uint4 v_ = (u_ < CPT - 1 || c_last) ? *reinterpret_cast<const uint4*>(Cbase + c_g[u_] + (k0)) \
-                                                : uint4{0, 0, 0, 0};                                     \
-      if constexpr (u_ < CH) c_lo[u_ < CH ? u_ : 0] = v_;                                                \
-      else c_hi[u_ < CH ? 0 : u_ - CH] = v_;                                                             \
-    });                                                                                                  \
-  } while (0)
-#define NOPT_LSTORE(buf)                                                                                 \
-  do {                                                                                                   \
-    int8_t* As_ = sm[buf];                                                                               \
-    if constexpr (!PK)                                                                                   \
-      _Pragma("unroll") for (int u = 0; u < APT; ++u) {                                                  \
-        const int e_ = t + NTH * u;                                                                      \
-        *reinterpret_cast<uint4*>(As_ + (e_ / ACQ) * AB + (((e_ % ACQ) / (4 * BMI)) * BMI + ar) * KS +   \
-                                  16 * swz(ar, ac)) = a_reg[u];                                          \
-      }                                                                                                  \
-    static_for<CPT>([&](auto U) {                                                                        \
-      constexpr int u_ = decltype(U)::value;                                                             \
-      uint4* d_ = reinterpret_cast<uint4*>(As_ + c_s[u_]);                                               \
-      if (u_ < CPT - 1 || c_last) {                                                                      \
-        if constexpr (u_ < CH) *d_ = c_lo[u_ < CH ? u_ : 0];                                             \
-        else *d_ = c_hi[u_ < CH ? 0 : u_ - CH];                                                          \
-      }                                                                                                  \
-    });                                                                                                  \
-  } while (0)
+  // slab k0 .. k0 + 63 of both operands (packed: of C) on its way into a stage
+  auto issue = [&](int k0, int8_t* dst) __attribute__((always_inline)) {
+    if constexpr (!PK)
+#pragma unroll
+      for (int u = 0; u < APT; ++u) load_lds16(rA[u], dst + 1024 * wu + 16 * NTH * u, avo, k0);
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) load_lds16(rC, dst + QPB * AB + 1024 * wu + 16 * NTH * u, cvo[u], k0);
+  };
   v4i_t acc[IT][JT][5];
 #pragma unroll
   for (int i = 0; i < IT; ++i)
@@ -683,10 +663,12 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
   if (have) {
     const int k0 = __builtin_ctz(todo) * KS;
     todo &= todo - 1u;
-    NOPT_GLOAD_A(k0);
-    if constexpr (PK) lstore_packed(sm[0]);
-    NOPT_GLOAD_C(k0);
-    NOPT_LSTORE(0);
+    issue(k0, sm[0]);
+    if constexpr (PK) {
+      gload_packed(k0);
+      lstore_packed(sm[0]);
+    }
+    lds_landed();
     __syncthreads();
   }
   const int lr = lane & 15, lc = lane >> 4;
@@ -694,9 +676,12 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
     const int cur = ks & 1;
     const bool more = todo != 0;
     const int kn = more ? __builtin_ctz(todo) * KS : 0;  // the next slab
-    // the B slab (HBM) is fetched before the products, the small C slab
-    // (L2-resident) after them (measured faster than fetching both first)
-    if (more) NOPT_GLOAD_A(kn);
+    // the next slab's loads all go out before the products (its stage was read
+    // in the previous round)
+    if (more) {
+      if constexpr (PK) gload_packed(kn);
+      issue(kn, sm[cur ^ 1]);
+    }
     const int8_t* As = sm[cur] + qq * AB;
     const int8_t* Cs = sm[cur] + QPB * AB;
     uint4 av[IT][4];
@@ -733,20 +718,13 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
       if constexpr (!PK && s_ + 1 < 4 * JT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       if constexpr (!PK) __builtin_amdgcn_sched_group_barrier(0x008, IT * (l < 2 ? 4 : 5 - l), 0);
     });
-    if (more) {
-      // packed: the B slab is converted and stored before the C slab is
-      // fetched (fewer registers live at once)
-      if constexpr (PK) lstore_packed(sm[cur ^ 1]);
-      NOPT_GLOAD_C(kn);
-      NOPT_LSTORE(cur ^ 1);
-    }
+    if constexpr (PK)
+      if (more) lstore_packed(sm[cur ^ 1]);
+    lds_landed();
     __syncthreads();
     todo &= todo - 1u;
     have = more;
   }
-#undef NOPT_GLOAD_A
-#undef NOPT_GLOAD_C
-#undef NOPT_LSTORE
   // X values in FP64 (rows m0 + rowl(i, v), columns colb(j) of the group)
   auto rowl = [&](int i, int v) { return wr * 16 * IT + i * 16 + 4 * lc + v; };
   auto colb = [&](int j) { return wc * 16 * JT + j * 16 + lr; };
