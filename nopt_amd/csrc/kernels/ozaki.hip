@@ -913,13 +913,30 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
     __syncthreads();
   }
 }
+// Block i of a half-transform over gx row tiles, gy groups of functions and gz
+// column groups, half_blocks() of them. Workgroups go to the 8 XCDs round
+// robin; all blocks of a function run on one XCD close in time, column group
+// fastest, so that the second column group of a tile, and in the packed form
+// the other row tiles of the triangle, find B in that XCD's L2, and the reads
+// of an XCD stay close together in memory. Against row tiles fastest over all
+// XCDs: one density of C20H42 1452 -> 1368 us, two of (H2O)13 863 -> 854, the
+// ragged batch of twelve clusters 5304 -> 5148 (a contiguous range of functions
+// per XCD instead of every eighth: 1374, 861, 5170).
+// False: a block beyond the last function.
+__device__ __forceinline__ bool half_vb(int i, int gx, int gy, int gz, VB* vb) {
+  const int j = i / 8, q = i % 8 + 8 * (j / (gx * gz));
+  *vb = VB{(j / gz) % gx, q, j % gz, gx, gy, gz};
+  return q < gy;
+}
 template <int NT, int WC, int NW, int QPB, int BMI, int WPE, bool PK>
-__global__ __launch_bounds__(64 * NW * QPB) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void k_half_i8(
+__global__ __launch_bounds__(64 * NW * QPB) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) void k_half_i8(int gx, int gy, int gz,
     const int8_t* __restrict__ Bd, long bplane, const int* __restrict__ Bp, long sq, const int8_t* __restrict__ Be8,
     const int* __restrict__ Be, const uint32_t* __restrict__ Bm, int nmb, long ld8, int nbf, int naux,
     const int8_t* __restrict__ Cd, long cplane, const int* __restrict__ Ce, double* __restrict__ X, long ldx,
     const XSplit xs) {
-  k_half_i8_body<NT, WC, NW, QPB, BMI, WPE, PK>(grid_vb(),
+  VB vb;
+  if (!half_vb((int)blockIdx.x, gx, gy, gz, &vb)) return;
+  k_half_i8_body<NT, WC, NW, QPB, BMI, WPE, PK>(vb,
       Bd, bplane, Bp, sq, Be8, Be, Bm, nmb, ld8, nbf, naux, Cd, cplane, Ce, X, ldx, xs);
 }
 template <int NT, int WC, int NW, int QPB, int BMI, int WPE, bool PK>
@@ -928,7 +945,9 @@ void k_half_i8_list(const ItemHalf* __restrict__ items,
     const int* __restrict__ first, int n) {
   const int i = list_item(first, n, (int)blockIdx.x);
   const ItemHalf& a = items[i];
-  k_half_i8_body<NT, WC, NW, QPB, BMI, WPE, PK>(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz),
+  VB vb;
+  if (!half_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz, &vb)) return;
+  k_half_i8_body<NT, WC, NW, QPB, BMI, WPE, PK>(vb,
       a.Bd, a.bplane, a.Bp, a.sq, a.Be8, a.Be, a.Bm, a.nmb, a.ld8, a.nbf, a.naux, a.Cd, a.cplane, a.Ce, a.X, a.ldx,
       a.xs);
 }
@@ -1616,6 +1635,9 @@ int half_i8_threads(int nt, int qpb, bool pk) {
   return 0;
 }
 
+// Blocks of a launch (half_vb).
+unsigned half_blocks(unsigned gx, unsigned gy, unsigned gz) { return 8 * ((gy + 7) / 8) * gx * gz; }
+
 template <typename T>
 void put_args(ListRec* r, const T& a) {
   r->args.resize(sizeof(T));
@@ -1629,11 +1651,10 @@ hipError_t launch_half_i8(int nt, int qpb, dim3 grid, hipStream_t s, const HalfB
   if (ce != hipSuccess) return ce;
 #define NOPT_HALF_I8(PK_, NT_, WC_, NW_, QPB_, BMI_, WPE_)                                                  \
   case half_cfg(PK_, NT_, QPB_):                                                                          \
-    k_half_i8<NT_, WC_, NW_, QPB_, BMI_, WPE_, PK_><<<dim3((nbf + BMI_ - 1) / BMI_, grid.y, grid.z),       \
-                                                     64 * NW_ * QPB_, 0, s>>>(b.Bd, b.bplane, b.Bp, b.sq,  \
-                                                                              b.Be8, b.Be, b.Bm, b.nmb, ld8, \
-                                                                              nbf, naux, Cd, cplane, Ce, X, \
-                                                                              ldx, xs);                     \
+    k_half_i8<NT_, WC_, NW_, QPB_, BMI_, WPE_, PK_>                                                       \
+        <<<half_blocks((nbf + BMI_ - 1) / BMI_, grid.y, grid.z), 64 * NW_ * QPB_, 0, s>>>(                 \
+            (nbf + BMI_ - 1) / BMI_, (int)grid.y, (int)grid.z, b.Bd, b.bplane, b.Bp, b.sq, b.Be8, b.Be,    \
+            b.Bm, b.nmb, ld8, nbf, naux, Cd, cplane, Ce, X, ldx, xs);                                      \
     break;
   switch (half_cfg(!b.Bd, nt, qpb)) {
     NOPT_HALF_CONFIGS(NOPT_HALF_I8)
@@ -1775,7 +1796,7 @@ hipError_t half_i8_item(int nt, int qpb, dim3 grid, const HalfB& b, long ld8, in
   const int gx = (nbf + bmi - 1) / bmi;
   r->kind = kListHalf;
   r->cfg = half_cfg(pk, nt, qpb);
-  r->blocks = gx * (int)grid.y * (int)grid.z;
+  r->blocks = (int)half_blocks(gx, grid.y, grid.z);
   r->threads = half_i8_threads(nt, qpb, pk);
   put_args(r, ItemHalf{b.Bd, b.bplane, b.Bp, b.sq, b.Be8, b.Be, b.Bm, b.nmb, ld8, nbf, naux, Cd, cplane, Ce, X, ldx,
                        xs, gx, (int)grid.y, (int)grid.z});
