@@ -1292,17 +1292,20 @@ constexpr int KT8 = 64;
 // the tiles of one split read the same X rows at about the same time, from
 // that XCD's L2. The grid is 1-D, ntiles * nsplit blocks; when that is not a
 // multiple of 8, the first (ntiles * nsplit) % 8 XCDs take one pair more.
-// BUF: the operand and exponent loads as buffer loads (32-bit offsets: a
-// digit plane and the exponents below 2^31 bytes, which the launchers check),
-// else as loads through 64-bit addresses.
-template <int NW, bool BUF>
+// The slabs go from memory straight into LDS: without the 32 registers a
+// thread staged them in, the Coulomb kernels of the second stream fit beside two
+// of its waves on a SIMD (192 of 512 registers each). With each class sum begun
+// by its first product instead of cleared: one density of C20H42 1378 -> 1335
+// us, two of (H2O)13 857 -> 830, the ragged batch of twelve clusters 5087 ->
+// 4927.
+template <int NW>
 __device__ __forceinline__ void k_syrk_i8_body(const VB vb, 
     const int8_t* __restrict__ Xd, long xplane, const int* __restrict__ Xe, long ldk, int nbf, int naux,
     int ntiles, int nsplit, double* __restrict__ Kpart) {
   // NW waves in a (NW/2) x 2 grid: each wave 64/(NW/2) rows (IT row tiles) x 32 columns
   constexpr int KS = 64, TB = 4 * KT8 * KS;  // bytes of one operand tile (4 planes)
-  constexpr int NTH = 64 * NW, IT = 64 / (NW / 2) / 16, OPT = 512 / NTH;  // operands loaded per thread
-  static_assert(IT >= 1 && OPT >= 1 && IT * 16 * (NW / 2) == 64, "tile split");
+  constexpr int NTH = 64 * NW, IT = 64 / (NW / 2) / 16;
+  static_assert(NTH == 256 && IT * 16 * (NW / 2) == 64, "tile split; a load per plane and operand tile");
   __shared__ __attribute__((aligned(16))) int8_t sm[2][2 * TB];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, wr = w >> 1, wc = w & 1;
   const int lr = lane & 15, lc = lane >> 4;
@@ -1314,72 +1317,31 @@ __device__ __forceinline__ void k_syrk_i8_body(const VB vb,
   const int q0 = (int)((long)naux * sp / ns), q1 = (int)((long)naux * (sp + 1) / ns);
   const int nkq = (int)(ldk / KS);  // k-slabs per auxiliary function
   const int nsl = (q1 - q0) * nkq;
-  // loader: row (t/4)%64 of operand tile (t/256 + o) (o < OPT; tile 0 rows
-  // bi, tile 1 rows bj), chunk t%4, all 4 planes
-  const int ar = (t >> 2) & 63, ac = t & 3, op0 = (OPT == 2) ? 0 : (t >> 8);
-  // rows beyond nbf load row nbf - 1 and store zeros: every lane issues the
-  // same loads, so that the waits count them exactly. Buffer form: a
-  // resource per digit plane, the lane's row and chunk as the vector offset,
-  // the slab's offset (the same for the whole block) as the scalar one.
-  __amdgpu_buffer_rsrc_t rX[4];
-  if constexpr (BUF)
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-      rX[p] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(Xd + p * xplane), (short)0, (int)xplane,
-                                                0x00020000);
-  long voff[OPT];
-  bool rok[OPT];
-#pragma unroll
-  for (int o = 0; o < OPT; ++o) {
-    const int m = ((op0 + o) == 0 ? bi : bj) * KT8 + ar;
-    rok[o] = m < nbf;
-    voff[o] = (long)min(m, nbf - 1) * ldk + 16 * ac;
-  }
+  // loader: a wave's load fills 1 KB of a plane of an operand tile (LDS chunk t:
+  // row t / 4, the swizzle in which chunk of it the lane asks for), wave w the
+  // rows 16 w .. 16 w + 15. Rows beyond nbf read row nbf - 1 (their outputs are
+  // never read). The resources start at the function (64-bit addresses; a function's rows are below 2 MB).
+  const int wu = __builtin_amdgcn_readfirstlane(w);
+  const int ar = t >> 2, ac = swz(ar, t & 3);
+  const int va = min(bi * KT8 + ar, nbf - 1) * (int)ldk + 16 * ac;
+  const int vc = min(bj * KT8 + ar, nbf - 1) * (int)ldk + 16 * ac;
   const long qstride = (long)nbf * ldk;
-  uint4 o_reg[OPT][4];
-  auto gload = [&](int sl) {
-    const int q = q0 + sl / nkq, k0 = (sl % nkq) * KS;
-    if constexpr (BUF) {
-      const int so = __builtin_amdgcn_readfirstlane((int)(q * qstride + k0));
+  auto issue = [&](int q, int k0, int8_t* dst) __attribute__((always_inline)) {
 #pragma unroll
-      for (int o = 0; o < OPT; ++o)
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          const auto x = __builtin_amdgcn_raw_buffer_load_b128(rX[p], (int)voff[o], so, 0);
-          o_reg[o][p] = uint4{x[0], x[1], x[2], x[3]};
-        }
-    } else {
-      const int8_t* base = Xd + q * qstride + k0;
-#pragma unroll
-      for (int o = 0; o < OPT; ++o)
-#pragma unroll
-        for (int p = 0; p < 4; ++p) o_reg[o][p] = *reinterpret_cast<const uint4*>(base + p * xplane + voff[o]);
-    }
-  };
-  auto lstore = [&](int buf) {
-#pragma unroll
-    for (int o = 0; o < OPT; ++o) {
-      int8_t* Ts = sm[buf] + (op0 + o) * TB;
-#pragma unroll
-      for (int p = 0; p < 4; ++p)
-        *reinterpret_cast<uint4*>(Ts + (p * KT8 + ar) * KS + 16 * swz(ar, ac)) =
-            rok[o] ? o_reg[o][p] : uint4{0, 0, 0, 0};
+    for (int p = 0; p < 4; ++p) {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<int8_t*>(Xd + p * xplane + q * qstride), (short)0, (int)qstride, 0x00020000);
+      load_lds16(r, dst + p * KT8 * KS + 1024 * wu, va, k0);
+      load_lds16(r, dst + TB + p * KT8 * KS + 1024 * wu, vc, k0);
     }
   };
   // exponents of this thread's accumulator rows (IT x 4) and columns (2)
   int ea[IT][4], eb[2];
-  __amdgpu_buffer_rsrc_t rXe;
-  if constexpr (BUF)
-    rXe = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(Xe), (short)0, (int)(4L * naux * nbf), 0x00020000);
   auto eload = [&](int q, int (&xa)[IT][4], int (&xb)[2]) {
-    // rows beyond nbf read row nbf - 1 (their products are zero)
-    auto ld = [&](int m) {
-      if constexpr (BUF)
-        return (int)__builtin_amdgcn_raw_buffer_load_b32(rXe, 4 * min(m, nbf - 1),
-                                                         __builtin_amdgcn_readfirstlane(4 * q * nbf), 0);
-      else
-        return Xe[(long)q * nbf + min(m, nbf - 1)];
-    };
+    // rows beyond nbf read row nbf - 1
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(Xe + (long)q * nbf), (short)0,
+                                                                       4 * nbf, 0x00020000);
+    auto ld = [&](int m) { return (int)__builtin_amdgcn_raw_buffer_load_b32(r, 4 * min(m, nbf - 1), 0, 0); };
 #pragma unroll
     for (int i = 0; i < IT; ++i)
 #pragma unroll
@@ -1397,29 +1359,30 @@ __device__ __forceinline__ void k_syrk_i8_body(const VB vb,
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       k64[i][j] = d4_t{0, 0, 0, 0};
-#pragma unroll
-      for (int c = 0; c < 5; ++c) acc[i][j][c] = v4i_t{0, 0, 0, 0};
     }
   if (nsl > 0) {
-    gload(0);
-    lstore(0);
+    issue(q0, 0, sm[0]);
+    lds_landed();
   }
   __syncthreads();
-  for (int sl = 0; sl < nsl; ++sl) {
+  for (int sl = 0, q = q0, kq = 0; sl < nsl; ++sl) {  // slab kq of function q
     const int cur = sl & 1;
-    const bool more = sl + 1 < nsl;
-    const bool qend = (sl % nkq) == nkq - 1;
+    const bool more = sl + 1 < nsl, qbeg = kq == 0, qend = kq == nkq - 1;
     // the exponents of this function's rows, needed after its last slab,
     // requested before the next slab, so that waiting for them leaves the
     // slab's loads in flight
-    if (qend) eload(q0 + sl / nkq, ea, eb);
+    if (qend) eload(q, ea, eb);
+    if (more) {
+      kq = qend ? 0 : kq + 1;
+      q += qend;
+    }
     // (the last slab loads itself again, unused: every path then issues
     // the same loads, and the wait for the exponents leaves the slab's in
     // flight)
-    gload(more ? sl + 1 : sl);
+    issue(q, kq * KS, sm[cur ^ 1]);
     const int8_t* As = sm[cur];
-    const int8_t* Bs = sm[cur] + TB;
-    if (!upper) {
+    const int8_t* Bs = As + TB;
+    auto products = [&](auto FIRST) __attribute__((always_inline)) {
       uint4 av[IT][4];
 #pragma unroll
       for (int i = 0; i < IT; ++i) {
@@ -1445,11 +1408,21 @@ __device__ __forceinline__ void k_syrk_i8_body(const VB vb,
         for (int i = 0; i < IT; ++i) {
           v4i_t* A = acc[i][j];
 #pragma unroll
-          for (int k = 0; k + l <= 4 && k < 4; ++k) A[k + l] = mfma_i8(av[i][k], bv, A[k + l]);
+          for (int k = 0; k + l <= 4 && k < 4; ++k) {
+            // the first product of a class in a function's first slab starts its sum
+            constexpr bool start = decltype(FIRST)::value;
+            A[k + l] = mfma_i8(av[i][k], bv, start && (l == 0 || (l == 1 && k == 3)) ? v4i_t{0, 0, 0, 0} : A[k + l]);
+          }
         }
         if constexpr (s_ + 1 < 8) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x008, IT * (l < 2 ? 4 : 5 - l), 0);
       });
+    };
+    if (!upper) {
+      if (qbeg)
+        products(std::true_type{});
+      else
+        products(std::false_type{});
       if (qend) {
         // combine the class sums of this auxiliary function: with |digit| <= 64
         // and ldk <= 1024, hi = 128 A0 + A1 and mid = 128 A2 + A3 are exact in
@@ -1465,12 +1438,10 @@ __device__ __forceinline__ void k_syrk_i8_body(const VB vb,
               const double sv = fma((double)hi, 0x1p21, fma((double)mid, 128.0, (double)A[4][v]));
               k64[i][j][v] += ldexp(sv, ea[i][v] + eb[j] - 40);
             }
-#pragma unroll
-            for (int c = 0; c < 5; ++c) A[c] = v4i_t{0, 0, 0, 0};
           }
       }
     }
-    if (more) lstore(cur ^ 1);
+    lds_landed();
     __syncthreads();
   }
   double* Kt = Kpart + ((long)sp * ntiles + tile) * KT8 * KT8;
@@ -1485,19 +1456,19 @@ __device__ __forceinline__ void k_syrk_i8_body(const VB vb,
         Kt[rr * KT8 + cc] = k64[i][j][v];
       }
 }
-template <int NW, bool BUF>
+template <int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2, NW / 2))) void k_syrk_i8(
     const int8_t* __restrict__ Xd, long xplane, const int* __restrict__ Xe, long ldk, int nbf, int naux,
     int ntiles, int nsplit, double* __restrict__ Kpart) {
-  k_syrk_i8_body<NW, BUF>(grid_vb(), Xd, xplane, Xe, ldk, nbf, naux, ntiles, nsplit, Kpart);
+  k_syrk_i8_body<NW>(grid_vb(), Xd, xplane, Xe, ldk, nbf, naux, ntiles, nsplit, Kpart);
 }
-template <int NW, bool BUF>
+template <int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 2, NW / 2)))
 void k_syrk_i8_list(const ItemSyrk* __restrict__ items,
     const int* __restrict__ first, int n) {
   const int i = list_item(first, n, (int)blockIdx.x);
   const ItemSyrk& a = items[i];
-  k_syrk_i8_body<NW, BUF>(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz),
+  k_syrk_i8_body<NW>(list_vb((int)blockIdx.x - first[i], a.gx, a.gy, a.gz),
       a.Xd, a.xplane, a.Xe, a.ldk, a.nbf, a.naux, a.ntiles, a.nsplit, a.Kpart);
 }
 
@@ -1838,14 +1809,11 @@ hipError_t jpart_slots_item(int nd, int nsplit, const int8_t* Bs, long splane, l
   return hipSuccess;
 }
 
-// the exchange's buffer-load form: 32-bit offsets cover a digit plane and the exponents
-bool syrk_buf(long xplane, int nbf, int naux) { return xplane <= 0x7fffffffL && 4L * naux * nbf <= 0x7fffffffL; }
-
 hipError_t syrk_i8_item(int ntiles, int nsplit, const int8_t* Xd, long xplane, const int* Xe, long ldk, int nbf,
                         int naux, double* Kpart, ListRec* r) {
   if (nsplit < 1 || ntiles <= 0 || ldk % 64 != 0 || ldk > 1024) return hipErrorInvalidValue;
   r->kind = kListSyrk;
-  r->cfg = syrk_buf(xplane, nbf, naux) ? 5 : 4;
+  r->cfg = 4;
   r->blocks = ntiles * nsplit;
   r->threads = 256;
   put_args(r, ItemSyrk{Xd, xplane, Xe, ldk, nbf, naux, ntiles, nsplit, Kpart, ntiles * nsplit, 1, 1});
@@ -1897,10 +1865,7 @@ hipError_t launch_list(int kind, int cfg, const void* items, const int* first, i
       break;
     }
     case kListSyrk:
-      if (cfg == 5)
-        k_syrk_i8_list<4, true><<<blocks, 256, 0, s>>>((const ItemSyrk*)items, first, n);
-      else
-        k_syrk_i8_list<4, false><<<blocks, 256, 0, s>>>((const ItemSyrk*)items, first, n);
+      k_syrk_i8_list<4><<<blocks, 256, 0, s>>>((const ItemSyrk*)items, first, n);
       break;
     default: return hipErrorInvalidValue;
   }
@@ -1911,12 +1876,7 @@ hipError_t launch_syrk_i8(int ntiles, int nsplit, hipStream_t s, const int8_t* X
                           long ldk, int nbf, int naux, double* Kpart) {
   if (nsplit < 1 || ntiles <= 0 || ldk % 64 != 0 || ldk > 1024) return hipErrorInvalidValue;
   // four waves of 32 x 32 (two waves per SIMD, two blocks per CU)
-  if (syrk_buf(xplane, nbf, naux))
-    k_syrk_i8<4, true><<<(unsigned)(ntiles * nsplit), 256, 0, s>>>(Xd, xplane, Xe, ldk, nbf, naux, ntiles, nsplit,
-                                                                    Kpart);
-  else
-    k_syrk_i8<4, false><<<(unsigned)(ntiles * nsplit), 256, 0, s>>>(Xd, xplane, Xe, ldk, nbf, naux, ntiles, nsplit,
-                                                                     Kpart);
+  k_syrk_i8<4><<<(unsigned)(ntiles * nsplit), 256, 0, s>>>(Xd, xplane, Xe, ldk, nbf, naux, ntiles, nsplit, Kpart);
   return hipGetLastError();
 }
 
