@@ -650,7 +650,15 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
   // in which the block's rows of B hold no nonzero digit (Bm: a 32-bit mask
   // per function and 32 rows); a zero slab adds nothing to the class sums,
   // so leaving it out changes no bit of X
-  const int nks = (int)(ld8 / KS);
+  // The slab of the diagonal comes first and is on its way before the masks are
+  // known; the row and column exponents of the epilogue are asked for here too
+  // (indices clamped into range; not in the packed form, which has no register
+  // to spare): a block lives for few slabs, and the waits for the masks and the
+  // exponents were a good part of its time (two densities of (H2O)13 822 -> 802 us,
+  // the ragged batch of twelve clusters 4921 -> 4849, C20H42 1331 -> 1323).
+  const int nks = (int)(ld8 / KS), kd = m0 / KS;
+  issue(kd * KS, sm[0]);
+  if constexpr (PK) gload_packed(kd * KS);
   uint32_t todo = nks >= 32 ? 0xffffffffu : (1u << nks) - 1u;
   if (Bm) {
     uint32_t any = 0;
@@ -663,24 +671,35 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
       }
     todo &= any;
   }
-  todo = __builtin_amdgcn_readfirstlane(todo);
-  bool have = todo != 0;
-  if (have) {
-    const int k0 = __builtin_ctz(todo) * KS;
-    todo &= todo - 1u;
-    issue(k0, sm[0]);
-    if constexpr (PK) {
-      gload_packed(k0);
-      lstore_packed(sm[0]);
-    }
-    lds_landed();
-    __syncthreads();
-  }
+  todo = __builtin_amdgcn_readfirstlane(todo & ~(1u << kd));
+  uint32_t sibling = PK ? 0u : todo & (1u << (kd ^ 1));
   const int lr = lane & 15, lc = lane >> 4;
-  for (int ks = 0; have; ++ks) {
+  // rows m0 + rowl(i, v), columns colb(j) of the group
+  auto rowl = [&](int i, int v) { return wr * 16 * IT + i * 16 + 4 * lc + v; };
+  auto colb = [&](int j) { return wc * 16 * JT + j * 16 + lr; };
+  int ebe[IT][4], ece[JT];
+  auto load_exponents = [&]() {
+    const long Qc = Q < naux ? Q : naux - 1;
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) ebe[i][v] = Be[Qc * nbf + min(m0 + rowl(i, v), nbf - 1)];
+#pragma unroll
+    for (int j = 0; j < JT; ++j) ece[j] = Ce[cg * BN + colb(j)];
+  };
+  if constexpr (PK)
+    lstore_packed(sm[0]);
+  else
+    load_exponents();
+  lds_landed();
+  __syncthreads();
+  for (int ks = 0;; ++ks) {
     const int cur = ks & 1;
+    // the next slab: the other half of the first one's 128-byte lines, then upwards
     const bool more = todo != 0;
-    const int kn = more ? __builtin_ctz(todo) * KS : 0;  // the next slab
+    const uint32_t pick = sibling ? sibling : todo & (0u - todo);
+    const int kn = more ? __builtin_ctz(pick) * KS : 0;
+    sibling = 0;
     // the next slab's loads all go out before the products (its stage was read
     // in the previous round)
     if (more) {
@@ -727,12 +746,9 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
       if (more) lstore_packed(sm[cur ^ 1]);
     lds_landed();
     __syncthreads();
-    todo &= todo - 1u;
-    have = more;
+    if (!more) break;
+    todo &= ~pick;
   }
-  // rows m0 + rowl(i, v), columns colb(j) of the group
-  auto rowl = [&](int i, int v) { return wr * 16 * IT + i * 16 + 4 * lc + v; };
-  auto colb = [&](int j) { return wc * 16 * JT + j * 16 + lr; };
   // a Q beyond naux holds zeros (rows beyond nbf are computed but never written)
   if (QPB > 1 && Q >= naux) {
 #pragma unroll
@@ -742,18 +758,7 @@ __device__ __forceinline__ void k_half_i8_body(const VB vb,
 #pragma unroll
         for (int c = 0; c < 5; ++c) acc[i][j][c] = v4i_t{0, 0, 0, 0};
   }
-  // the row and column exponents, all loads issued at once (indices clamped
-  // into range)
-  int ebe[IT][4], ece[JT];
-  {
-    const long Qc = Q < naux ? Q : naux - 1;
-#pragma unroll
-    for (int i = 0; i < IT; ++i)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) ebe[i][v] = Be[Qc * nbf + min(m0 + rowl(i, v), nbf - 1)];
-#pragma unroll
-    for (int j = 0; j < JT; ++j) ece[j] = Ce[cg * BN + colb(j)];
-  }
+  if constexpr (PK) load_exponents();
   // S = 2^28 x the digit sum, X = S 2^(em + ec - 40): hi = 128 A0 + A1 is exact
   // in int32 (|A0| <= 4096 ld8, ld8 <= 2048), so is mid = 128 A2 + A3 for
   // ld8 <= 1024 (|A2| <= 3 * 4096 ld8), and every partial sum below 2^52 is
