@@ -442,7 +442,8 @@ __global__ __launch_bounds__(256) void k_syrk_f32(const float* __restrict__ X, l
 // reads in flight each, and the four sums are added in the order p = 0..3, so
 // that the result is reproducible. (One thread per element over all splits,
 // one read after the other, took 32 us for the 116 partials of a 24-function
-// K and 46 us for 103 partials at 490 functions; this takes 4 and 28 us.)
+// K and 46 us for 103 partials at 490 functions; this takes 4 and, for the 28
+// partials there now, 10 us.)
 struct ItemFin {
   const double* Jpart;
   int nsj;
@@ -835,12 +836,14 @@ int order_out(nopt_jk_ctx* c, hipStream_t s) {
 // Q-splits of the integer Coulomb pair: about four blocks per CU over the
 // slots the kernels walk. At most 32 J partials, which the output sums; 64 where
 // 32 would leave half of the CUs without a block (three waters, 72 functions: J
-// 13.3 -> 10.7 us, the output 6.3 -> 6.6).
+// 13.3 -> 10.7 us, the output 6.3 -> 6.6) and X's digit planes, at most 4 naux
+// nbf (nbf + 64) bytes, leave ample room for the partials in the static scratch.
 void coulomb_split_defaults(nopt_jk_ctx* c) {
   const int nsb = nopt::gamma_slot_blocks(c->nlslots);
   const int nbj = (c->nlslots + 256 * nopt::kJSPL - 1) / (256 * nopt::kJSPL);
   c->nsg = (int)std::max(1L, std::min(c->naux, (4L * c->ncu + nsb - 1) / nsb));
-  c->nsj8 = (int)std::max(1L, std::min({c->naux, nbj <= 4 ? 64L : 32L, (4L * c->ncu + nbj - 1) / nbj}));
+  const bool small = nbj <= 4 && 4.0 * c->naux * c->nbf * (c->nbf + 64) <= (double)((size_t)128 << 20);
+  c->nsj8 = (int)std::max(1L, std::min({c->naux, small ? 64L : 32L, (4L * c->ncu + nbj - 1) / nbj}));
 }
 
 // Once B's integer forms are written: the Coulomb segments and slots that
