@@ -171,6 +171,87 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
   }
 }
 
+// ---------------------------------------------------------------- Coulomb
+// Jpart[d][s][m][n] = sum_{Q in split s} gamma[d][Q] B[Q][m][n] over the lower
+// triangle, for ND densities at once (B is read once). A block owns the row
+// pair (p, nbf-1-p): nbf+1 elements, read as aligned pairs of columns (a
+// row's last pair may include its first upper element, which lies inside the
+// row because ld > nbf and is not written). The Q loop is unrolled so that UNR
+// loads per thread are in flight. gamma[d*gstride + Q], or with grows > 0 its
+// partials as the FP64 half-transform leaves them (launch_half_f64).
+template <int ND>
+__device__ __forceinline__ void k_jpart_body(int p, int s, double* gs /* ND x the longest split */,
+                                             const double* __restrict__ B, long ld, int nbf, int naux,
+                                             const double* __restrict__ gamma, long gstride, int grows, int ns,
+                                             double* __restrict__ Jpart, long jstride) {
+  constexpr int UNR = ND == 1 ? 8 : 4;
+  const int q0 = (int)((long)naux * s / ns), q1 = (int)((long)naux * (s + 1) / ns);
+  const int len = q1 - q0;
+  for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x)
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const double* gd = gamma + d * gstride + q;
+      double v = 0.0;
+      if (grows > 0) {  // partials of the FP64 half-transform: one per tile of grows rows that holds rows of q
+        const long r = (long)q * nbf;
+        const int t1 = (int)((r + nbf - 1) / grows);
+#pragma unroll 4
+        for (int tl = (int)(r / grows); tl <= t1; ++tl) v += gd[tl];
+      } else {
+        v = gd[0];
+      }
+      gs[d * len + q - q0] = v;
+    }
+  __syncthreads();
+  auto g = [&](int d, int i) { return gs[d * len + i]; };
+  const int m1 = p, m2 = nbf - 1 - p;
+  const int s1 = (m1 + 2) / 2, s2 = (m2 != m1) ? (m2 + 2) / 2 : 0;
+  const long qstride = (long)nbf * ld;
+  for (int slot = threadIdx.x; slot < s1 + s2; slot += blockDim.x) {
+    const int row = slot < s1 ? m1 : m2;
+    const int col = 2 * (slot < s1 ? slot : slot - s1);
+    const double* bp = B + (long)q0 * qstride + (long)row * ld + col;
+    double a0[ND], a1[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) a0[d] = a1[d] = 0.0;
+    int q = q0;
+    for (; q + UNR <= q1; q += UNR) {
+      double2 v[UNR];
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) v[u] = *reinterpret_cast<const double2*>(bp + (long)u * qstride);
+#pragma unroll
+      for (int u = 0; u < UNR; ++u)
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+          a0[d] += g(d, q - q0 + u) * v[u].x;
+          a1[d] += g(d, q - q0 + u) * v[u].y;
+        }
+      bp += (long)UNR * qstride;
+    }
+    for (; q < q1; ++q) {
+      const double2 v = *reinterpret_cast<const double2*>(bp);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        a0[d] += g(d, q - q0) * v.x;
+        a1[d] += g(d, q - q0) * v.y;
+      }
+      bp += qstride;
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      double* Js = Jpart + d * jstride + (long)s * nbf * nbf;
+      Js[(long)row * nbf + col] = a0[d];
+      if (col + 1 <= row) Js[(long)row * nbf + col + 1] = a1[d];
+    }
+  }
+}
+template <int ND>
+__global__ __launch_bounds__(256) void k_jpart(JF64 a) {
+  extern __shared__ double gs[];
+  k_jpart_body<ND>(blockIdx.x, blockIdx.y, gs, a.B, a.ld, a.nbf, a.naux, a.gamma, a.gstride, a.grows, a.nsplit,
+                   a.Jpart, a.jstride);
+}
+
 // ------------------------------------------------------------------ exchange
 // Tiles of 64 x 64 with four waves of 32 x 32, four blocks per CU. The
 // contraction runs over (Q, orbital) as one index, kpad orbitals per function
@@ -194,9 +275,8 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
 // without LDS or barriers, takes 0.94 instead of 0.98 ms alone at 84 orbitals,
 // but 1.5 instead of 1.3 ms beside the J pass. Four blocks per CU: with two,
 // or a barrier every 8 or 32 orbitals, it is 5-15 % slower.
-__global__ __launch_bounds__(256, 4) void k_syrk_f64(const double* __restrict__ X, long ldx, int nbf, int naux,
-                                                     int kpad, int ntiles, int nsplit,
-                                                     double* __restrict__ Kpart) {
+__device__ __forceinline__ void k_syrk_f64_body(const double* __restrict__ X, long ldx, int nbf, int naux, int kpad,
+                                                int ntiles, int nsplit, double* __restrict__ Kpart) {
   constexpr int T = kSyrkF64Tile;
   __shared__ __attribute__((aligned(16))) double sm[2][2][T][18];
   const int t = threadIdx.x, lane = t & 63, lr = lane & 15, g = lane >> 4;
@@ -282,6 +362,27 @@ __global__ __launch_bounds__(256, 4) void k_syrk_f64(const double* __restrict__ 
 #pragma unroll
       for (int v = 0; v < 4; ++v)
         Kt[(wr + i * 16 + acc_row<double>(lane, v)) * T + wc + j * 16 + lr] = acc[i][j][v];
+}
+__global__ __launch_bounds__(256, 4) void k_syrk_f64(const double* __restrict__ X, long ldx, int nbf, int naux,
+                                                     int kpad, int ntiles, int nsplit,
+                                                     double* __restrict__ Kpart) {
+  k_syrk_f64_body(X, ldx, nbf, naux, kpad, ntiles, nsplit, Kpart);
+}
+// The exchange, and behind its blocks the J pass in the same launch: the two do
+// not depend on each other, one is bound by the matrix unit and the other by
+// memory, and a launch of its own costs a small build more than its J pass
+// takes (one water molecule 27.1 -> 23.2 us).
+template <int ND>
+__global__ __launch_bounds__(256, 4) void k_syrk_j_f64(const double* __restrict__ X, long ldx, int nbf, int naux,
+                                                       int kpad, int ntiles, int nsplit, double* __restrict__ Kpart,
+                                                       JF64 a) {
+  __shared__ double gs[kRideGamma];
+  const int b = (int)blockIdx.x - ntiles * nsplit, np = (a.nbf + 1) / 2;
+  if (b < 0)
+    k_syrk_f64_body(X, ldx, nbf, naux, kpad, ntiles, nsplit, Kpart);
+  else
+    k_jpart_body<ND>(b % np, b / np, gs, a.B, a.ld, a.nbf, a.naux, a.gamma, a.gstride, a.grows, a.nsplit, a.Jpart,
+                     a.jstride);
 }
 
 // ---------------------------------------------------- active-space integrals
@@ -440,12 +541,36 @@ int syrk_f64_splits(int nsplit, int naux, int kpad) {
   return (int)std::max(1L, std::min((long)nsplit, (long)naux * kpad / 32));
 }
 
+hipError_t launch_jpart_f64(const JF64& a, int nd, hipStream_t s) {
+  const dim3 grid((a.nbf + 1) / 2, a.nsplit);
+  const size_t lds = sizeof(double) * nd * ((a.naux + a.nsplit - 1) / a.nsplit);
+  switch (nd) {
+    case 1: k_jpart<1><<<grid, 256, lds, s>>>(a); break;
+    case 2: k_jpart<2><<<grid, 256, lds, s>>>(a); break;
+    case 3: k_jpart<3><<<grid, 256, lds, s>>>(a); break;
+    case 4: k_jpart<4><<<grid, 256, lds, s>>>(a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+bool jpart_rides_f64(int nd, int naux, int nsplit) {
+  return nd >= 1 && nd <= 2 && (long)nd * ((naux + nsplit - 1) / nsplit) <= kRideGamma;
+}
+
 hipError_t launch_syrk_f64(int ntiles, int nsplit, hipStream_t s, const double* X, long ldx, int nbf, int naux,
-                           int kpad, double* Kpart) {
+                           int kpad, double* Kpart, const JF64* j, int nd) {
   const int kt = (nbf + kSyrkF64Tile - 1) / kSyrkF64Tile;
   if (nsplit < 1 || nsplit > naux || ntiles != kt * (kt + 1) / 2 || kpad < 4 || kpad % 4 || kpad > ldx || ldx % 2 || (reinterpret_cast<uintptr_t>(X) & 15))
     return hipErrorInvalidValue;
-  k_syrk_f64<<<(unsigned)(ntiles * nsplit), 256, 0, s>>>(X, ldx, nbf, naux, kpad, ntiles, nsplit, Kpart);
+  if (j && !jpart_rides_f64(nd, j->naux, j->nsplit)) return hipErrorInvalidValue;
+  const unsigned nx = (unsigned)(ntiles * nsplit), njb = j ? (unsigned)((j->nbf + 1) / 2 * j->nsplit) : 0u;
+  if (!j)
+    k_syrk_f64<<<nx, 256, 0, s>>>(X, ldx, nbf, naux, kpad, ntiles, nsplit, Kpart);
+  else if (nd == 1)
+    k_syrk_j_f64<1><<<nx + njb, 256, 0, s>>>(X, ldx, nbf, naux, kpad, ntiles, nsplit, Kpart, *j);
+  else
+    k_syrk_j_f64<2><<<nx + njb, 256, 0, s>>>(X, ldx, nbf, naux, kpad, ntiles, nsplit, Kpart, *j);
   return hipGetLastError();
 }
 

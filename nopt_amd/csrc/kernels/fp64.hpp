@@ -31,6 +31,27 @@ constexpr int kActiveGroup = 32;
 hipError_t launch_active_half(hipStream_t s, const double* B, long ld, int nbf, int naux, const double* Cp, int ldc,
                               int na, double* R);
 
+// The J pass over FP64 rows: Jpart[d*jstride + (s*nbf + m)*nbf + n], n <= m, the
+// sum over the functions Q of split s of gamma_d[Q] B[Q][m][n] (ld > nbf).
+// gamma[d*gstride + Q], or with grows > 0 the partials of launch_half_f64
+// (tiles of grows rows). launch_jpart_f64: up to four densities, nd*ceil(naux /
+// nsplit) gamma values in LDS (at most 64 KB). jpart_rides_f64: whether the
+// pass can go into the launch of an exchange: up to two densities, and a split's
+// gamma values in what four exchange blocks leave of a CU's LDS.
+struct JF64 {
+  const double* B;
+  long ld;
+  int nbf, naux;
+  const double* gamma;
+  long gstride;
+  int grows, nsplit;
+  double* Jpart;
+  long jstride;
+};
+constexpr int kRideGamma = 320;
+hipError_t launch_jpart_f64(const JF64& a, int nd, hipStream_t s);
+bool jpart_rides_f64(int nd, int naux, int nsplit);
+
 constexpr int kSyrkF64Tile = 64;  // exchange tile edge
 
 // Kpart[split][tile][r][c] = sum over the split's functions Q of
@@ -42,6 +63,7 @@ constexpr int kSyrkF64Tile = 64;  // exchange tile edge
 // shorter one is over before its loads pay, and its partial tile has to be
 // summed).
 int syrk_f64_splits(int nsplit, int naux, int kpad);
+// With j also the J pass of j's nd densities (jpart_rides_f64) in the same launch.
 hipError_t launch_syrk_f64(int ntiles, int nsplit, hipStream_t s, const double* X, long ldx, int nbf, int naux,
-                           int kpad, double* Kpart);
+                           int kpad, double* Kpart, const JF64* j = nullptr, int nd = 0);
 }  // namespace nopt

@@ -266,82 +266,6 @@ __global__ void k_gamma(const double* __restrict__ gpart, int mtiles, int naux,
   gamma[Q] = s;
 }
 
-// ---------------------------------------------------------------- Coulomb
-// Jpart[d][s][m][n] = sum_{Q in split s} gamma[d][Q] B[Q][m][n] over the lower
-// triangle, for ND densities at once (B is read once). A block owns the row
-// pair (p, nbf-1-p): nbf+1 elements, read as aligned pairs of columns (a
-// row's last pair may include its first upper element, which lies inside the
-// row because ld > nbf and is not written). The Q loop is unrolled so that UNR
-// loads per thread are in flight. gamma[d*gstride + Q], or with grows > 0 its
-// partials as the FP64 half-transform leaves them (launch_half_f64).
-template <int ND>
-__global__ __launch_bounds__(256) void k_jpart(const double* __restrict__ B, long ld, int nbf, int naux,
-                                               const double* __restrict__ gamma, long gstride, int grows,
-                                               double* __restrict__ Jpart, long jstride) {
-  constexpr int UNR = ND == 1 ? 8 : 4;
-  extern __shared__ double gs[];  // ND x the longest split
-  const int p = blockIdx.x, s = blockIdx.y, ns = gridDim.y;
-  const int q0 = (int)((long)naux * s / ns), q1 = (int)((long)naux * (s + 1) / ns);
-  const int len = q1 - q0;
-  for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x)
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      const double* gd = gamma + d * gstride + q;
-      double v = 0.0;
-      if (grows > 0) {  // partials of the FP64 half-transform: one per tile of grows rows that holds rows of q
-        const long r = (long)q * nbf;
-        const int t1 = (int)((r + nbf - 1) / grows);
-#pragma unroll 4
-        for (int tl = (int)(r / grows); tl <= t1; ++tl) v += gd[tl];
-      } else {
-        v = gd[0];
-      }
-      gs[d * len + q - q0] = v;
-    }
-  __syncthreads();
-  auto g = [&](int d, int i) { return gs[d * len + i]; };
-  const int m1 = p, m2 = nbf - 1 - p;
-  const int s1 = (m1 + 2) / 2, s2 = (m2 != m1) ? (m2 + 2) / 2 : 0;
-  const long qstride = (long)nbf * ld;
-  for (int slot = threadIdx.x; slot < s1 + s2; slot += blockDim.x) {
-    const int row = slot < s1 ? m1 : m2;
-    const int col = 2 * (slot < s1 ? slot : slot - s1);
-    const double* bp = B + (long)q0 * qstride + (long)row * ld + col;
-    double a0[ND], a1[ND];
-#pragma unroll
-    for (int d = 0; d < ND; ++d) a0[d] = a1[d] = 0.0;
-    int q = q0;
-    for (; q + UNR <= q1; q += UNR) {
-      double2 v[UNR];
-#pragma unroll
-      for (int u = 0; u < UNR; ++u) v[u] = *reinterpret_cast<const double2*>(bp + (long)u * qstride);
-#pragma unroll
-      for (int u = 0; u < UNR; ++u)
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          a0[d] += g(d, q - q0 + u) * v[u].x;
-          a1[d] += g(d, q - q0 + u) * v[u].y;
-        }
-      bp += (long)UNR * qstride;
-    }
-    for (; q < q1; ++q) {
-      const double2 v = *reinterpret_cast<const double2*>(bp);
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        a0[d] += g(d, q - q0) * v.x;
-        a1[d] += g(d, q - q0) * v.y;
-      }
-      bp += qstride;
-    }
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-      double* Js = Jpart + d * jstride + (long)s * nbf * nbf;
-      Js[(long)row * nbf + col] = a0[d];
-      if (col + 1 <= row) Js[(long)row * nbf + col + 1] = a1[d];
-    }
-  }
-}
-
 // --------------------------------------------------------------- exchange
 // Kpart[s][tile][r][c] = sum_{Q in split s} sum_i X[Q][bi*KT+r][i] X[Q][bj*KT+c][i]
 // (FP32 mode): FP32 chains of 16 terms, added in FP64.
@@ -683,8 +607,9 @@ struct nopt_jk_ctx {
 
 namespace {
 // largest triangle of B (in FP64, times the densities) of which a build runs in
-// line on one stream
-constexpr size_t kInlineBytes = (size_t)64 << 20;
+// line on one stream (enqueue_batch): FP64 and integer builds whose J pass rides
+// on the exchange's launch, and the others
+constexpr size_t kInlineF64 = (size_t)1 << 30, kInlineI8 = (size_t)288 << 20, kInlineOther = (size_t)64 << 20;
 constexpr int kPhases = 6;  // staging, half-transform, gamma, J partials, exchange, J output
 constexpr int kTimedBuilds = 512;
 }  // namespace
@@ -1365,14 +1290,20 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   // run on the side stream, forked after the staging (after the
   // half-transform in the integer mode, or when gamma rides on it) and joined
   // before the build ends, so that they overlap the exchange.
-  // A small build runs in line instead: its Coulomb pair is over sooner than
-  // the second stream has taken it up and been waited for (two hops of about
-  // 10 us), and J and K of a density leave in one launch. Water clusters, one
-  // density, microseconds in line and with the second stream: 24 functions 26
-  // and 63 (FP64), 31 and 52 (int8), 96 functions 46 and 59, 55 and 70, 144
-  // functions 93 and 97, 87 and 100, 192 functions 174 and 168, 153 and 159;
-  // two densities cross at about half that size.
-  const bool inl = !rec && !tm && sizeof(double) * (double)naux * (double)c->npair * std::max(nj, 1) <= (double)kInlineBytes;
+  // A smaller build runs in line instead: the second stream takes about 10 us to
+  // be taken up and as long to be waited for, J and K of a density leave in one
+  // launch, and the J pass goes into the launch of the first exchange, where it
+  // reads memory beside the matrix products all the same. In line and with the
+  // second stream, microseconds, FP64: 96 functions 44 and 59, 192 functions 156
+  // and 172, 250 functions 329 and 345, 346 functions 995 and 1015, 394 functions
+  // 1612 and 1625, 490 functions 3154 and 3000; int8: 96 functions 45 and 70, 192
+  // functions 139 and 151, 240 functions 240 and 240, 288 functions 384 and 376;
+  // two densities cross at half the triangle.
+  const int nsb = i8 && nj && !rec ? nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj) : 0;
+  const bool jrides = !rec && anyK && nj > 0 &&
+                      (f64 ? nopt::jpart_rides_f64(nj, naux, nsj) : i8 && nopt::jpart_rides_i8(nj, naux, nsj, nsb));
+  const size_t inline_bytes = !jrides ? kInlineOther : f64 ? kInlineF64 : kInlineI8;
+  const bool inl = !rec && !tm && sizeof(double) * (double)naux * (double)c->npair * std::max(nj, 1) <= (double)inline_bytes;
   const bool overlap = !rec && !tm && nj > 0 && anyK && !inl;
   const dim3 gfin((unsigned)((nbf + kFinCols - 1) / kFinCols), (unsigned)nbf);  // output blocks
   // the integer mode works on the functions in the order of B's integer
@@ -1425,7 +1356,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     } else if (i8) {
       CHK_(nopt::launch_gamma_slots(nj, c->nsg, sj, c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lslots,
                                     c->nlslots, c->lsegs, c->nlseg, w.Dp, ldb, c->dstride, w.gslot,
-                                    nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj) ? nullptr : w.gamma,
+                                    nsb ? nullptr : w.gamma,
                                     naux));
     } else {
 #define NOPT_GF(ND)                                                                                         \
@@ -1439,6 +1370,13 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     cmark(3);
     return hipSuccess;
   };
+  const nopt::JF64 jf64{c->B64, c->ld64, nbf, naux, f64 && fused ? w.gpart : w.gamma,
+                        f64 && fused ? nopt::half_f64_gstride(naux, nbf) : (long)naux,
+                        f64 && fused ? nopt::kHalfF64Rows : 0, nsj, Jpart, (long)nsj * nn};
+  const nopt::ItemJ ji8{c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lsegs, c->nlseg,
+                        nsb ? w.gslot : w.gamma, naux, Jpart, (long)nsj * nn, (c->nlseg + 255) / 256, nsj, 1};
+  // in line, the J pass goes into the launch of the first exchange
+  bool jwait = false;
   auto coulomb_j = [&]() -> hipError_t {
     if (i8 && rec) {
       nopt::ListRec r;
@@ -1447,23 +1385,11 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       rec->add(5, r);
       return hipSuccess;
     }
-    if (i8) {
-      const int nsb = nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj);
+    if (i8)
       return nopt::launch_jpart_slots(nj, nsj, sj, c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lslots,
                                       c->nlslots, c->lsegs, c->nlseg, nsb ? w.gslot : w.gamma, naux, nsb, Jpart,
                                       (long)nsj * nn);
-    }
-    dim3 gj((nbf + 1) / 2, nsj);
-    const size_t jlds = sizeof(double) * nj * ((naux + nsj - 1) / nsj);  // at most JCHUNK_MAX values
-#define NOPT_JP(ND)                                                                                     \
-  case ND:                                                                                              \
-    k_jpart<ND><<<gj, 256, jlds, sj>>>(c->B64, c->ld64, nbf, naux, f64 && fused ? w.gpart : w.gamma,         \
-                                       f64 && fused ? nopt::half_f64_gstride(naux, nbf) : (long)naux,      \
-                                       f64 && fused ? nopt::kHalfF64Rows : 0, Jpart, (long)nsj * nn);      \
-    break;
-    switch (nj) { NOPT_JP(1) NOPT_JP(2) NOPT_JP(3) NOPT_JP(4) }
-#undef NOPT_JP
-    return hipGetLastError();
+    return nopt::launch_jpart_f64(jf64, nj, sj);
   };
   auto coulomb = [&]() -> hipError_t {
     CHK_(coulomb_gamma());
@@ -1589,7 +1515,11 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     HIPCHK(coulomb_out());
     coulomb_at = 1;
   }
-  if (coulomb_at == 2) HIPCHK(coulomb());
+  if (coulomb_at == 2) {
+    HIPCHK(coulomb_gamma());
+    jwait = inl && jrides;
+    if (!jwait) HIPCHK(coulomb_j());
+  }
   mark(4);
   // K of density d, in line together with its J
   auto out_k = [&](int d, const double* Kp, int nsk_, int ntl, int kt) {
@@ -1627,7 +1557,9 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
             HIPCHK(nopt::syrk_i8_item(c->ntiles8, c->nsk8, xd, rowsq * ldk, xe, ldk, nbf, (int)npq, kp, &r));
             rec->add(7, r);
           } else {
-            HIPCHK(nopt::launch_syrk_i8(c->ntiles8, c->nsk8, s, xd, rowsq * ldk, xe, ldk, nbf, (int)npq, kp));
+            HIPCHK(nopt::launch_syrk_i8(c->ntiles8, c->nsk8, s, xd, rowsq * ldk, xe, ldk, nbf, (int)npq, kp,
+                                        jwait ? &ji8 : nullptr, nj, nsb));
+            jwait = false;
           }
         }
       } else {
@@ -1635,7 +1567,8 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
         HIPCHK(nopt::split_rows_i8((const double*)w.X + off[d], ldx, (int)it[d].nocc, rows, 4, (int8_t*)w.Xd, ldk,
                                    rows, rows * ldk, (int*)w.Xe, s));
         HIPCHK(nopt::launch_syrk_i8(c->ntiles8, c->nsk8, s, (const int8_t*)w.Xd, rows * ldk, (const int*)w.Xe, ldk,
-                                    nbf, (int)naux, w.Kpart));
+                                    nbf, (int)naux, w.Kpart, jwait ? &ji8 : nullptr, nj, nsb));
+        jwait = false;
       }
       out_k(d, w.Kpart + kfirst * kseg, nsum * c->nsk8, c->ntiles8, nopt::kSyrkI8Tile);
     } else {
@@ -1643,17 +1576,20 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       const int ntl = f64 ? c->ntiles8 : c->ntiles;
       dim3 gk(ntl, ns);
       if (f64)
-        HIPCHK(nopt::launch_syrk_f64(ntl, ns, s, (const double*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart));
+        HIPCHK(nopt::launch_syrk_f64(ntl, ns, s, (const double*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart,
+                                     jwait ? &jf64 : nullptr, nj));
       else if (prec == NOPT_PREC_FP32)
         k_syrk_f32<<<gk, 256, 0, s>>>((const float*)w.X + off[d], ldx, nbf, naux, kpad, w.Kpart);
       else
         HIPCHK(nopt::launch_syrk_bf16(prec == NOPT_PREC_BF16X3 ? 2 : 3, gk, s, (const float*)w.X + off[d], ldx,
                                       nbf, naux, kpad, w.Kpart));
+      jwait = false;
       out_k(d, w.Kpart, ns, ntl, f64 ? nopt::kSyrkF64Tile : KT);
     }
     HIPCHK(hipGetLastError());
   }
   mark(5);
+  if (jwait) HIPCHK(coulomb_j());  // there was no exchange
   if (coulomb_at == 2) HIPCHK(coulomb_out());
   if (overlap) {
     HIPCHK(hipEventRecord(c->ev_join, c->side));

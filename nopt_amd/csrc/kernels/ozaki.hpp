@@ -162,10 +162,15 @@ hipError_t launch_jpart_slots(int nd, int nsplit, hipStream_t s, const int8_t* B
 
 // Exchange partials over 64x64 lower-triangle tiles: Kpart[split][tile] for
 // ntiles tiles and nsplit Q-splits (each XCD a contiguous range of the
-// (tile, split) pairs).
-constexpr int kSyrkI8Tile = 64;
+// (tile, split) pairs). With j also the J pass of launch_jpart_slots in the same
+// launch, for up to two densities (jpart_rides_i8: the gamma sums of a split fit
+// beside the exchange's LDS).
+constexpr int kSyrkI8Tile = 64, kRideGammaI8 = 512;
+struct ItemJ;
+bool jpart_rides_i8(int nd, int naux, int nsplit, int nsb);
 hipError_t launch_syrk_i8(int ntiles, int nsplit, hipStream_t s, const int8_t* Xd, long xplane, const int* Xe,
-                          long ldk, int nbf, int naux, double* Kpart);
+                          long ldk, int nbf, int naux, double* Kpart, const ItemJ* j = nullptr, int nd = 0,
+                          int nsb = 0);
 
 // Work lists (common.hpp): the kernels above can run the grids of several
 // systems in one launch. A ListRec is one item: the kernel (kind and template
