@@ -11,36 +11,40 @@ namespace nopt {
 namespace {
 
 // ------------------------------------------------------------ half-transform
-// X[r][c] = sum_n B[r][n] C[c][n] over the rows r = Q*nbf + m of all functions
-// as one range (no padding of the rows of a function), and with ND > 0 the
-// partial sums of gamma_d[Q] = sum_mn B[Q][m][n] D_d[m][n].
+// X[r][c] = sum_n B[r][n] C[c][n] over the rows r = Q*nbf + m of all functions,
+// taken as pair rows (row m of the functions 2p and 2p + 1) in one range p*nbf + m
+// without padding of the rows of a pair, and with ND > 0 the partial sums of
+// gamma_d[Q] = sum_mn B[Q][m][n] D_d[m][n].
 //
-// A block takes 128 rows and 16 NT columns, a wave 32 rows of them. Only C
-// passes through LDS (all four waves read it; slabs of 16, double buffered,
+// A block takes 64 pair rows and 16 NT columns, a wave 16 pair rows of them. Only
+// C passes through LDS (all four waves read it; slabs of 16, double buffered,
 // one barrier per slab of 16 NT products per wave); a wave's rows of B go
 // straight from global memory to its registers, a row's 16 values of a slab in
 // two loads back to back, so that the second finds its line in the L1, and are
-// requested again for the next slab as soon as their products are issued. The
-// rows of D follow those of B. The order of the terms is free: in a step of
+// requested again for the next slab as soon as their products are issued. Row m
+// of D serves both functions of the pair: with rows of one function, as many
+// loads and registers went to D as to B. The order of the terms is free: in a step of
 // eight, lane l holds the terms 2 (l / 16) and 2 (l / 16) + 1 of row l % 16 of
 // either operand, the first for one product, the second for the next.
 //
 // At C20H42 (490 functions, 2366 auxiliary functions, 81 orbitals, one
 // density) 1.80 ms, 51 TFLOP/s of useful products (61 as issued: 96 columns),
 // against 2.85 ms with B and C staged through LDS by loads of 64-byte lane
-// stride in 128-row tiles per function; 1.69 ms without the density, whose rows
-// cost registers (two waves per SIMD instead of three). With up to three
-// column tiles it runs at the rate of B's reads (1.0-1.1 ms here). One row of
-// D per function of four waves through LDS, extra columns by vector
-// instructions and wave tiles of 16, 48 or 64 rows were slower.
+// stride in 128-row tiles per function; 1.69 ms without the density. With up to
+// four column tiles it runs at the rate of B's reads, and the pairs tell: the
+// gradient at 298 functions and 49 orbitals 640 -> 593 us, two densities of 192
+// functions 274 -> 264, the host call at 250 functions and 41 orbitals 474 -> 456.
+// Four waves per SIMD where 128 registers (nearly) hold the kernel, up to three
+// column tiles and one density: that call 455 -> 440 us with four against three.
+// Extra columns by vector instructions and wave tiles of 16, 48 or 64 rows were slower.
 //
 // The column groups of a row tile are consecutive blocks of one XCD, so that
-// the second finds B in its L2. gpart[d*gstride + tile + Q] is the part of
-// gamma_d[Q] in row tile `tile` (consecutive (tile, Q) pairs that share rows
-// have consecutive sums tile + Q).
-constexpr int kHalfRows = kHalfF64Rows;
+// the second finds B in its L2. gpart[d*gstride + 2*(tile + p) + i] is the part
+// of gamma_d[2p + i] in row tile `tile` (consecutive (tile, pair)s that share
+// rows have consecutive sums tile + p).
+constexpr int kHalfRows = kHalfF64Rows;  // pair rows
 template <int NT, int ND, int OCC>
-__global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict__ B, long ld, long rows, int nbf,
+__global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict__ B, long ld, int naux, int nbf,
                                                        const double* __restrict__ Cp, const double* __restrict__ Dp,
                                                        long dstride, double* __restrict__ X, int ldx,
                                                        double* __restrict__ gpart, long gstride, int ntile,
@@ -50,18 +54,24 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
   const int t = threadIdx.x, lane = t & 63, lr = lane & 15, g = lane >> 4, w = t >> 6;
   const int local = blockIdx.x / 8, cg = local % groups, tile = (local / groups) * 8 + (int)(blockIdx.x % 8);
   if (tile >= ntile) return;
-  const long rb = (long)tile * kHalfRows;  // the block's first row
-  const char* Bb = reinterpret_cast<const char*>(B + rb * ld);
+  const long rb = (long)tile * kHalfRows, prows = (long)((naux + 1) / 2) * nbf;  // pair rows: the block's first, all
+  const long p0 = rb / nbf;
+  const int m0 = (int)(rb % nbf);
+  // row of function i of the pair of pair row rb + x, counted from (2 p0, m0);
+  // of an odd last function's missing partner that function's (not written)
+  auto row_of = [&](int x, int i) {
+    const int p = (m0 + x) / nbf, m = (m0 + x) % nbf;
+    return (2 * p + (2 * (p0 + p) + i < naux ? i : 0)) * nbf + m - m0;
+  };
+  const char* Bb = reinterpret_cast<const char*>(B + (2 * p0 * nbf + m0) * ld);
   const char* Db = reinterpret_cast<const char*>(Dp);
   const char* Cb = reinterpret_cast<const char*>(Cp);
-  // byte offsets of the lane's rows (beyond the last row: that row again, not written)
-  unsigned ao[MI], dof[MI];
+  // byte offsets of the lane's rows (beyond the last pair row: that one again, not written)
+  const int xr = (int)min((long)(w * 16 + lr), prows - 1 - rb);
+  unsigned ao[MI];
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int r = (int)min((long)((w * MI + i) * 16 + lr), rows - 1 - rb);
-    ao[i] = 8u * (unsigned)(r * (int)ld + 2 * g);
-    dof[i] = 8u * (unsigned)((int)((rb + r) % nbf) * (int)ld + 2 * g);
-  }
+  for (int i = 0; i < MI; ++i) ao[i] = 8u * ((unsigned)row_of(xr, i) * (unsigned)ld + 2u * g);
+  const unsigned dof = 8u * ((unsigned)((m0 + xr) % nbf) * (unsigned)ld + 2u * g);
   // C loader: 16-byte chunk e % 8 of column e / 8 (a column beyond ldx repeats the last one, not written)
   unsigned co[CPT];
 #pragma unroll
@@ -69,14 +79,16 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
     const int e = min(t + 256 * u, NC * 8 - 1);
     co[u] = 8u * (unsigned)(min(cg * NC + (e >> 3), ldx - 1) * (int)ld + 2 * (e & 7));
   }
-  d2_t a[MI][2], d[ND ? MI : 1][ND ? ND : 1][2], cr[CPT];
+  d2_t a[MI][2], d[ND ? ND : 1][2], cr[CPT];
   auto aload = [&](int i, long k) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      a[i][h] = *reinterpret_cast<const d2_t*>(Bb + 8 * k + ao[i] + 64 * h);
+    for (int h = 0; h < 2; ++h) a[i][h] = *reinterpret_cast<const d2_t*>(Bb + 8 * k + ao[i] + 64 * h);
+    if (i == MI - 1) {  // both rows' terms with the old ones are done
 #pragma unroll
-      for (int q = 0; q < ND; ++q)
-        d[i][q][h] = *reinterpret_cast<const d2_t*>(Db + 8 * (q * dstride + k) + dof[i] + 64 * h);
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < ND; ++q)
+          d[q][h] = *reinterpret_cast<const d2_t*>(Db + 8 * (q * dstride + k) + dof + 64 * h);
     }
   };
   auto cload = [&](long k) {
@@ -121,7 +133,7 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
           for (int j = 0; j < NT; ++j) acc[i][j] = mfma_f64(a[i][h][e], cc[j][e], acc[i][j]);
 #pragma unroll
         for (int q = 0; q < ND; ++q)
-          rd[i][q] = fma(a[i][h][1], d[i][q][h][1], fma(a[i][h][0], d[i][q][h][0], rd[i][q]));
+          rd[i][q] = fma(a[i][h][1], d[q][h][1], fma(a[i][h][0], d[q][h][0], rd[i][q]));
       }
       aload(i, kn);
       // keeps the operand reads of the next rows, and their registers, behind these products
@@ -131,20 +143,21 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int v = 0; v < 4; ++v) {
+    const int x = w * 16 + acc_row<double>(lane, v);
+    if (rb + x >= prows) continue;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const long r = rb + (w * MI + i) * 16 + acc_row<double>(lane, v);
-      if (r < rows) {
-        double* xr = X + r * ldx + cg * NC;
+    for (int i = 0; i < MI; ++i) {
+      if (i && 2 * (p0 + (m0 + x) / nbf) + i >= naux) continue;
+      double* xo = X + (2 * p0 * nbf + m0 + row_of(x, i)) * ldx + cg * NC;
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-          if (cg * NC + j * 16 + lr < ldx) xr[j * 16 + lr] = acc[i][j][v];
-      }
+      for (int j = 0; j < NT; ++j)
+        if (cg * NC + j * 16 + lr < ldx) xo[j * 16 + lr] = acc[i][j][v];
     }
+  }
   if constexpr (ND > 0) {
     if (cg != 0) return;
-    double(*red)[kHalfRows] = reinterpret_cast<double(*)[kHalfRows]>(&sm[0][0][0]);
+    double(*red)[MI][kHalfRows] = reinterpret_cast<double(*)[MI][kHalfRows]>(&sm[0][0][0]);
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -152,21 +165,21 @@ __global__ __launch_bounds__(256, OCC) void k_half_f64(const double* __restrict_
         double x = rd[i][q];
         x += __shfl_xor(x, 16, 64);
         x += __shfl_xor(x, 32, 64);
-        if (g == 0) red[q][(w * MI + i) * 16 + lr] = x;
+        if (g == 0) red[q][i][w * 16 + lr] = x;
       }
     __syncthreads();
-    // a wave per function: its rows inside the tile
-    const long re = min(rb + kHalfRows, rows);
-    const int Q0 = (int)(rb / nbf), Q1 = (int)((re - 1) / nbf);
-    for (int Q = Q0 + w; Q <= Q1; Q += 4) {
-      const int lo = (int)(max((long)Q * nbf, rb) - rb), hi = (int)(min((long)(Q + 1) * nbf, re) - rb);
+    // a wave per pair of functions: its rows inside the tile, one per lane
+    static_assert(kHalfRows == 64, "a lane per pair row");
+    const int xe = (int)min((long)kHalfRows, prows - rb), np = (m0 + xe - 1) / nbf;  // the tile's rows, its last pair
+    for (int p = w; p <= np; p += 4) {
+      const bool in = lane < xe && (m0 + lane) / nbf == p;
 #pragma unroll
-      for (int q = 0; q < ND; ++q) {
-        double x = 0.0;
-        for (int r = lane; r < kHalfRows; r += 64) x += r >= lo && r < hi ? red[q][r] : 0.0;
-        x = warp_sum(x);
-        if (lane == 0) gpart[q * gstride + tile + Q] = x;
-      }
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int q = 0; q < ND; ++q) {
+          const double x = warp_sum(in ? red[q][i][lane] : 0.0);
+          if (lane == 0) gpart[q * gstride + 2 * (tile + p0 + p) + i] = x;
+        }
     }
   }
 }
@@ -190,13 +203,13 @@ __device__ __forceinline__ void k_jpart_body(int p, int s, double* gs /* ND x th
   for (int q = q0 + threadIdx.x; q < q1; q += blockDim.x)
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
-      const double* gd = gamma + d * gstride + q;
+        const double* gd = gamma + d * gstride + q;  // (2 (q / 2) + q % 2)
       double v = 0.0;
-      if (grows > 0) {  // partials of the FP64 half-transform: one per tile of grows rows that holds rows of q
-        const long r = (long)q * nbf;
+      if (grows > 0) {  // partials of the FP64 half-transform: one per tile of grows pair rows that holds rows of q
+        const long r = (long)(q / 2) * nbf;
         const int t1 = (int)((r + nbf - 1) / grows);
 #pragma unroll 4
-        for (int tl = (int)(r / grows); tl <= t1; ++tl) v += gd[tl];
+        for (int tl = (int)(r / grows); tl <= t1; ++tl) v += gd[2 * tl];
       } else {
         v = gd[0];
       }
@@ -500,16 +513,15 @@ int half_f64_nt(long ncol, int* groups) {
 
 hipError_t launch_half_f64(int nt, int groups, int nd, hipStream_t s, const double* B, long ld, int naux, int nbf,
                            const double* Cp, const double* Dp, long dstride, double* X, long ldx, double* gpart) {
-  const long rows = (long)naux * nbf;
   const int ntile = half_f64_tiles(naux, nbf);
   if (nd < 0 || nd > kHalfF64Dens || groups < 1 || 16L * nt * groups < ldx || 16L * nt * (groups - 1) >= ldx ||
-      ldx % 2 || ld % 16 || ld < nbf || (nd && (!Dp || !gpart)) || ld * std::max(ldx, (long)kHalfF64Rows) > 1L << 28 ||
-      ld * nbf > 1L << 28)
+      ldx % 2 || ld % 16 || ld < nbf || (nd && (!Dp || !gpart)) || ld * std::max(ldx, 2L * kHalfF64Rows) > 1L << 28 ||
+      ld * (nbf + kHalfF64Rows) >= 1L << 28)
     return hipErrorInvalidValue;
   const unsigned grid = (unsigned)((ntile + 7) / 8 * 8 * groups);
 #define NOPT_HALF_F64(NT_, ND_)                                                                                  \
   if (nt == NT_ && nd == ND_)                                                                                    \
-    k_half_f64<NT_, ND_, (NT_ <= 4 && ND_ < 2 ? 3 : 2)><<<grid, 256, 0, s>>>(B, ld, rows, nbf, Cp, Dp, dstride, X, (int)ldx, \
+    k_half_f64<NT_, ND_, (NT_ <= 3 && ND_ < 2 ? 4 : NT_ <= 4 ? 3 : 2)><<<grid, 256, 0, s>>>(B, ld, naux, nbf, Cp, Dp, dstride, X, (int)ldx, \
                                                                  gpart, half_f64_gstride(naux, nbf), ntile, groups);
 #define NOPT_HALF_F64_ND(NT_) NOPT_HALF_F64(NT_, 0) NOPT_HALF_F64(NT_, 1) NOPT_HALF_F64(NT_, 2)
   NOPT_HALF_F64_ND(1)

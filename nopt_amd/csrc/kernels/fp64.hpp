@@ -9,14 +9,15 @@ namespace nopt {
 // all naux functions and c < ldx (an even count; column groups of 16 nt,
 // half_f64_nt picks nt and their number), B's and Cp's columns nbf.. up to the
 // next multiple of 16 zero. With nd > 0 also the gamma partials of the nd
-// densities Dp + d*dstride (rows of ld): those of gamma_d[Q] are
-// gpart[d*gstride + tile + Q] for the tiles of kHalfF64Rows rows that hold
-// rows of Q, tile = Q*nbf / kHalfF64Rows .. (Q*nbf + nbf - 1) / kHalfF64Rows.
-constexpr int kHalfF64Rows = 128, kHalfF64Dens = 2;
+// densities Dp + d*dstride (rows of ld), per tile of kHalfF64Rows pair rows (row
+// m of the functions 2p and 2p + 1: pair row p*nbf + m): those of gamma_d[Q], p
+// = Q / 2, are gpart[d*gstride + 2*(tile + p) + Q % 2] for the tiles that hold
+// rows of the pair, tile = p*nbf / kHalfF64Rows .. (p*nbf + nbf - 1) / kHalfF64Rows.
+constexpr int kHalfF64Rows = 64, kHalfF64Dens = 2;
 static inline int half_f64_tiles(long naux, long nbf) {
-  return (int)((naux * nbf + kHalfF64Rows - 1) / kHalfF64Rows);
+  return (int)(((naux + 1) / 2 * nbf + kHalfF64Rows - 1) / kHalfF64Rows);
 }
-static inline long half_f64_gstride(long naux, long nbf) { return half_f64_tiles(naux, nbf) + naux; }
+static inline long half_f64_gstride(long naux, long nbf) { return 2 * (half_f64_tiles(naux, nbf) + (naux + 1) / 2); }
 int half_f64_nt(long ncol, int* groups);
 hipError_t launch_half_f64(int nt, int groups, int nd, hipStream_t s, const double* B, long ld, int naux, int nbf,
                            const double* Cp, const double* Dp, long dstride, double* X, long ldx, double* gpart);
