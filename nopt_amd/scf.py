@@ -25,6 +25,17 @@ class SCFResult(dict):
     __getattr__ = dict.__getitem__
 
 
+def fix_signs(C):
+    """C with each column's sign such that its first component within 1e-6 of
+    its largest magnitude is positive. LAPACK's signs change with the rounding
+    of the matrix; what starts from these orbitals with a build that rounds as
+    coarsely as the integer mode (a CASSCF taken down to that mode's gradient
+    noise) goes another way for other signs, and should not for rounding."""
+    a = np.abs(C)
+    first = (a > (1.0 - 1e-6) * a.max(axis=0)).argmax(axis=0)
+    return C * np.where(C[first, np.arange(C.shape[1])] < 0.0, -1.0, 1.0)
+
+
 def rhf(mol, ctx=None, prec="fp64", switch_err=1e-5, e_conv=1e-10, d_conv=1e-8, max_it=100,
         diis_size=8, verbose=False, H=None, S=None, switch_ctx=None):
     """Returns SCFResult(E, C (nbf x nbf, columns are MOs), eps, D, F, iters,
@@ -94,7 +105,7 @@ def rhf(mol, ctx=None, prec="fp64", switch_err=1e-5, e_conv=1e-10, d_conv=1e-8, 
             C = X @ Cp
         # converged only on an FP64 iteration: a run that switches to the FP64
         # end-game at its last iteration has not refined its energy
-        return SCFResult(E=E, C=C, eps=eps, D=D, F=F, H=H, S=S, iters=it, builds=builds, history=hist,
+        return SCFResult(E=E, C=fix_signs(C), eps=eps, D=D, F=F, H=H, S=S, iters=it, builds=builds, history=hist,
                          converged=bool(done and built == "fp64"), switch_iter=switch_iter)
     finally:
         if own:
