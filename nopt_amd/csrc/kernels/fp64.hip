@@ -28,7 +28,7 @@ namespace {
 // either operand, the first for one product, the second for the next.
 //
 // At C20H42 (490 functions, 2366 auxiliary functions, 81 orbitals, one
-// density) 1.80 ms, 51 TFLOP/s of useful products (61 as issued: 96 columns),
+// density) 1.75 ms, 53 TFLOP/s of useful products (62 as issued: 96 columns),
 // against 2.85 ms with B and C staged through LDS by loads of 64-byte lane
 // stride in 128-row tiles per function; 1.69 ms without the density. With up to
 // four column tiles it runs at the rate of B's reads, and the pairs tell: the
