@@ -932,17 +932,21 @@ int form_B(nopt_jk_ctx* c, const double* host, const double* dL, const double* d
   auto prepare_forms = [&]() -> int {
     int r = NOPT_OK;
     c->b_ready = false;
-    if (keep64 && !c->B64) r = dev_alloc((void**)&c->B64, sizeof(double) * rows * c->ld64, "B (FP64)");
-    if (!r && keep8 && !c->Be) {
-      if (c->bfull) r = dev_alloc((void**)&c->Bd, (size_t)4 * rows * c->ld8, "B digit planes");
-      if (!r) r = dev_alloc((void**)&c->Be, sizeof(int) * rows, "B row exponents");
-      if (!r) r = dev_alloc((void**)&c->Be8, (size_t)na * c->ld8, "B row exponents (bytes)");
+    // each by its own pointer: where one could not be had, the next call asks for what is missing
+    auto need = [&](auto*& p, size_t bytes, const char* what) {
+      if (!r && !p) r = dev_alloc((void**)&p, bytes, what);
+    };
+    if (keep64) need(c->B64, sizeof(double) * rows * c->ld64, "B (FP64)");
+    if (keep8) {
+      if (c->bfull) need(c->Bd, (size_t)4 * rows * c->ld8, "B digit planes");
+      need(c->Be, sizeof(int) * rows, "B row exponents");
+      need(c->Be8, (size_t)na * c->ld8, "B row exponents (bytes)");
       c->splane = na * 16L * c->nseg;
-      if (!r) r = dev_alloc((void**)&c->Bs, (size_t)5 * c->splane, "packed lower triangle of B");
+      need(c->Bs, (size_t)5 * c->splane, "packed lower triangle of B");
       c->nmb = (int)((nbf + 31) / 32);
-      if (!r && c->ld8 <= 2048) r = dev_alloc((void**)&c->Bm, sizeof(uint32_t) * na * c->nmb, "slab masks of B");
-      if (!r) r = dev_alloc((void**)&c->perm, sizeof(int) * nbf, "order of the functions");
-      if (!r) r = dev_alloc((void**)&c->pinv, sizeof(int) * nbf, "inverse order of the functions");
+      if (c->ld8 <= 2048) need(c->Bm, sizeof(uint32_t) * na * c->nmb, "slab masks of B");
+      need(c->perm, sizeof(int) * nbf, "order of the functions");
+      need(c->pinv, sizeof(int) * nbf, "inverse order of the functions");
     }
     if (r) return r;
     if (keep64) HIPCHK(hipMemsetAsync(c->B64, 0, sizeof(double) * rows * c->ld64, s));
