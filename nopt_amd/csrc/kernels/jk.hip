@@ -650,6 +650,16 @@ void dev_free(P*& p) {
   p = nullptr;
 }
 
+constexpr long kEnergyParts = 1024;  // partial sums of the energy
+// values of the two buffers of gamma partials: by row tile (or pair of
+// functions and row tile, two densities) and by block of Coulomb slots
+long gpart_count(const nopt_jk_ctx* c) {
+  return std::max(c->naux * c->mtiles64, nopt::kHalfF64Dens * nopt::half_f64_gstride(c->naux, c->nbf));
+}
+long gslot_count(const nopt_jk_ctx* c) {
+  return (long)nopt::gamma_partial_blocks(c->nslots, c->nseg) * kMaxBatch * c->naux;
+}
+
 void free_ring(nopt_jk_ctx* c) {
   for (int b = 0; b < 2; ++b) {
     if (c->ring[b]) (void)hipHostFree(c->ring[b]);
@@ -1731,11 +1741,7 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
     return set_error(NOPT_EHIP, std::string("nopt_jk_create: ") + hip_msg(e));
   }
   const long nn = nbf * nbf;
-  if (!rc)
-    rc = dev_alloc((void**)&c->gpart,
-                   sizeof(double) * std::max(naux * c->mtiles64,
-                                             nopt::kHalfF64Dens * nopt::half_f64_gstride(naux, nbf)),
-                   "gamma partials");
+  if (!rc) rc = dev_alloc((void**)&c->gpart, sizeof(double) * gpart_count(c), "gamma partials");
   if (!rc) rc = dev_alloc((void**)&c->gamma, sizeof(double) * kMaxBatch * naux, "gamma");
   if (!rc) {
     static_assert(nopt::kSyrkI8Tile == nopt::kSyrkF64Tile, "ntiles8 counts the tiles of both");
@@ -1751,7 +1757,7 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
   if (!rc) rc = dev_alloc((void**)&c->dD, sizeof(double) * nn, "D");
   if (!rc) rc = dev_alloc((void**)&c->dH, sizeof(double) * nn, "H");
   if (!rc) rc = dev_alloc((void**)&c->dF, sizeof(double) * nn, "F");
-  if (!rc) rc = dev_alloc((void**)&c->epart, sizeof(double) * 1024, "energy partials");
+  if (!rc) rc = dev_alloc((void**)&c->epart, sizeof(double) * kEnergyParts, "energy partials");
   if (!rc) rc = dev_alloc((void**)&c->dE, sizeof(double), "energy");
   if (!rc) rc = dev_alloc((void**)&c->info, sizeof(int), "info");
   if (!rc) {
@@ -1773,10 +1779,7 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
     if (!rc) rc = dev_alloc((void**)&c->lslots, sizeof(int) * c->nslots, "Coulomb live slot table");
     if (!rc) rc = dev_alloc((void**)&c->lsegs, sizeof(int) * c->nseg, "Coulomb live segment table");
     if (!rc) rc = dev_alloc((void**)&c->jlive, ones.size(), "Coulomb live slot map");
-    if (!rc)
-      rc = dev_alloc((void**)&c->gslot,
-                     sizeof(double) * nopt::gamma_partial_blocks(c->nslots, c->nseg) * kMaxBatch * naux,
-                     "gamma partials");
+    if (!rc) rc = dev_alloc((void**)&c->gslot, sizeof(double) * gslot_count(c), "gamma partials");
     c->nlseg = c->nseg;
     if (!rc && (hipMemcpy(c->slots, tab.data(), sizeof(int) * c->nslots, hipMemcpyHostToDevice) != hipSuccess ||
                 hipMemcpy(c->segs, stab.data(), sizeof(int) * c->nseg, hipMemcpyHostToDevice) != hipSuccess ||
@@ -2248,15 +2251,28 @@ int nopt_jk_zero_blocks(const nopt_jk_ctx* c, double out[3]) {
 
 long nopt_jk_device_bytes(const nopt_jk_ctx* c) {
   if (!c) return 0;
-  long b = 0;
-  if (c->B64) b += sizeof(double) * c->naux * c->nbf * c->ld64;
-  if (c->Bd) b += 4L * c->naux * c->nbf * c->ld8;
-  if (c->Bs) b += sizeof(int) * c->naux * c->nbf + c->naux * c->ld8 + 5L * c->splane;
-  if (c->Bm) b += sizeof(uint32_t) * c->naux * c->nmb;
+  const long nn = c->nbf * c->nbf, rows = c->naux * c->nbf;
+  long b = 0;     // bytes
+  long d = 0;     // FP64 values
+  long i = 0;     // 32-bit values
+  // made by create
+  d += gpart_count(c) + gslot_count(c) + kMaxBatch * (c->naux + c->dstride) + 5 * nn + kEnergyParts + 1;
+  i += 1 + 2L * (c->nslots + c->nseg);
+  b += c->nbf * c->nsr;
+  // the kept forms of B
+  if (c->B64) d += rows * c->ld64;
+  if (c->Bd) b += 4 * rows * c->ld8;
+  if (c->Be) i += rows;
+  if (c->Be8) b += c->naux * c->ld8;
+  if (c->Bs) b += 5 * c->splane;
+  if (c->Bm) i += c->naux * c->nmb;
+  i += c->nbf * ((c->perm ? 1 : 0) + (c->pinv ? 1 : 0));
+  // grown by builds and the host entry points
   b += (long)(c->X_bytes + c->Cp_bytes + c->Cd_bytes + c->Ce_bytes + c->Xd_bytes + c->Xe_bytes + c->Jpart_bytes);
   b += (long)(c->Kpart_bytes + c->act_bytes);
-  b += sizeof(double) * (c->naux * c->mtiles64 + kMaxBatch * c->naux + kMaxBatch * c->dstride + 5 * c->nbf * c->nbf);
-  return b;
+  d += c->dC_cap + (c->dG ? nn : 0);
+  for (int k = 0; k < kMaxBatch - 1; ++k) d += c->xD_cap[k] + c->xC_cap[k] + c->xJ_cap[k] + c->xK_cap[k];
+  return b + (long)sizeof(double) * d + (long)sizeof(int) * i;
 }
 
 int nopt_jk_build_device(nopt_jk_ctx* c, const double* dD, const double* dC, long nocc, double* dJ,
@@ -2607,7 +2623,7 @@ int nopt_jk_fock_energy(nopt_jk_ctx* c, const double* H, const double* D, const 
   HIPCHK(hipMemcpyAsync(c->dD, D, sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
   if (J) HIPCHK(hipMemcpyAsync(c->dJ, J, sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
   if (K) HIPCHK(hipMemcpyAsync(c->dK, K, sizeof(double) * nn, hipMemcpyHostToDevice, c->stream));
-  const int nblk = (int)std::min<long>(1024, (nn + 255) / 256);
+  const int nblk = (int)std::min(kEnergyParts, (nn + 255) / 256);
   k_fock_energy<<<nblk, 256, 0, c->stream>>>(c->dH, c->dD, J ? c->dJ : nullptr, K ? c->dK : nullptr, cj, ck,
                                              nn, c->dF, c->epart);
   k_sum<<<1, 256, 0, c->stream>>>(c->epart, nblk, c->dE);
@@ -2631,7 +2647,7 @@ int enqueue_energy_gradient(nopt_jk_ctx* c, const double* dH, const double* dC, 
   HIPCHK(hipGetLastError());
   int rc = enqueue_build(c, c->dD, dC, nocc, c->dJ, c->dK, prec, s);
   if (rc) return rc;
-  const int nblk = (int)std::min<long>(1024, (nn + 255) / 256);
+  const int nblk = (int)std::min(kEnergyParts, (nn + 255) / 256);
   k_fock_energy<<<nblk, 256, 0, s>>>(dH, c->dD, c->dJ, c->dK, 2.0, 1.0, nn, F, c->epart);
   k_sum<<<1, 256, 0, s>>>(c->epart, nblk, dE);
   HIPCHK(hipGetLastError());

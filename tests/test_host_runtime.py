@@ -28,3 +28,7 @@ def run(tmp_path_factory):
 
 def test_failed_allocation_and_retry(run):
     run("host_alloc_retry")
+
+
+def test_device_bytes_are_those_held(run):
+    run("host_device_bytes")
