@@ -225,7 +225,9 @@ int nopt_jk_energy_gradient_device(nopt_jk_ctx* ctx, const double* dH, const dou
  * gamma cache allows, at least 16), integer exchange splits, integer gamma
  * splits, integer J splits, and where the integer Coulomb
  * pair starts on its side stream: 0 after the half-transform, 1 gamma beside
- * the half-transform and J after it, 2 both beside it}. create picks them from the
+ * the half-transform and J after it, 2 both beside it; builds of up to 288 MB
+ * of B's triangle times densities use no side stream, and the tuner leaves this
+ * entry as it is for them}. create picks them from the
  * device's CU count; nopt_jk_autotune times `reps` device builds of (dD, dC)
  * in mode `prec` on `stream` for each candidate of each split count in turn
  * (two rounds of coordinate descent), keeps the fastest and returns its mean

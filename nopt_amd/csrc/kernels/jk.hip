@@ -1177,6 +1177,35 @@ struct Rec {
   void add(int phase, const nopt::ListRec& r) { items.push_back(RecItem{phase, r}); }
 };
 
+// How a build of nj densities with J (nsj J splits) goes: nsb > 0 when its J
+// pass adds the gamma partials (of nsb slot blocks), jrides when the pass can go
+// into the launch of the first exchange, inl when the build runs in line on one
+// stream instead of with its Coulomb pair on the second.
+// The second stream takes about 10 us to be taken up and as long to be waited
+// for; in line, J and K of a density leave in one launch, and the J pass goes
+// into the launch of the first exchange, where it reads memory beside the matrix
+// products all the same. In line and with the second stream, microseconds, FP64:
+// 96 functions 44 and 59, 192 functions 156 and 172, 250 functions 329 and 345,
+// 346 functions 995 and 1015, 394 functions 1612 and 1625, 490 functions 3154
+// and 3000; int8: 96 functions 45 and 70, 192 functions 139 and 151, 240
+// functions 240 and 240, 288 functions 384 and 376; two densities cross at half
+// the triangle.
+struct Route {
+  int nsb = 0;
+  bool jrides = false, inl = false;
+};
+Route route_of(const nopt_jk_ctx* c, int prec, int nj, int nsj, bool anyK) {
+  const bool f64 = prec == NOPT_PREC_FP64, i8 = prec == NOPT_PREC_INT8;
+  const int naux = (int)c->naux;
+  Route r;
+  if (i8 && nj) r.nsb = nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj);
+  r.jrides = anyK && nj > 0 &&
+             (f64 ? nopt::jpart_rides_f64(nj, naux, nsj) : i8 && nopt::jpart_rides_i8(nj, naux, nsj, r.nsb));
+  const size_t limit = !r.jrides ? kInlineOther : f64 ? kInlineF64 : kInlineI8;
+  r.inl = sizeof(double) * (double)c->naux * (double)c->npair * std::max(nj, 1) <= (double)limit;
+  return r;
+}
+
 // With rec, the integer build is recorded instead of enqueued (no timing, no
 // side stream; the fused exchange split only).
 int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStream_t s, void* work_area = nullptr,
@@ -1304,20 +1333,11 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
   // run on the side stream, forked after the staging (after the
   // half-transform in the integer mode, or when gamma rides on it) and joined
   // before the build ends, so that they overlap the exchange.
-  // A smaller build runs in line instead: the second stream takes about 10 us to
-  // be taken up and as long to be waited for, J and K of a density leave in one
-  // launch, and the J pass goes into the launch of the first exchange, where it
-  // reads memory beside the matrix products all the same. In line and with the
-  // second stream, microseconds, FP64: 96 functions 44 and 59, 192 functions 156
-  // and 172, 250 functions 329 and 345, 346 functions 995 and 1015, 394 functions
-  // 1612 and 1625, 490 functions 3154 and 3000; int8: 96 functions 45 and 70, 192
-  // functions 139 and 151, 240 functions 240 and 240, 288 functions 384 and 376;
-  // two densities cross at half the triangle.
-  const int nsb = i8 && nj && !rec ? nopt::gamma_slots_unsummed(nj, c->nlslots, c->nlseg, naux, nsj) : 0;
-  const bool jrides = !rec && anyK && nj > 0 &&
-                      (f64 ? nopt::jpart_rides_f64(nj, naux, nsj) : i8 && nopt::jpart_rides_i8(nj, naux, nsj, nsb));
-  const size_t inline_bytes = !jrides ? kInlineOther : f64 ? kInlineF64 : kInlineI8;
-  const bool inl = !rec && !tm && sizeof(double) * (double)naux * (double)c->npair * std::max(nj, 1) <= (double)inline_bytes;
+  // A smaller build runs in line instead (route_of).
+  const Route route = rec ? Route{} : route_of(c, prec, nj, nsj, anyK);
+  const int nsb = route.nsb;
+  const bool jrides = route.jrides;
+  const bool inl = !tm && route.inl;
   const bool overlap = !rec && !tm && nj > 0 && anyK && !inl;
   const dim3 gfin((unsigned)((nbf + kFinCols - 1) / kFinCols), (unsigned)nbf);  // output blocks
   // the integer mode works on the functions in the order of B's integer
@@ -1963,6 +1983,8 @@ int nopt_jk_autotune(nopt_jk_ctx* c, const double* dD, const double* dC, long no
   rc = measure(&best);
   for (int round = 0; round < 2 && !rc; ++round)
     for (int k = 0; k < nk && !rc; ++k) {
+      // (where the Coulomb pair starts on the second stream: of no effect on a build in line)
+      if (knobs[k] == &c->cplace && (nocc < 1 || route_of(c, prec, 1, c->nsj8, true).inl)) continue;
       int keep = *knobs[k];
       for (int v : cand[k]) {
         if (v == keep) continue;

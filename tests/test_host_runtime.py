@@ -32,3 +32,7 @@ def test_failed_allocation_and_retry(run):
 
 def test_device_bytes_are_those_held(run):
     run("host_device_bytes")
+
+
+def test_autotuner_leaves_unused_settings(run):
+    run("host_autotune")
