@@ -221,7 +221,10 @@ int nopt_jk_energy_gradient_device(nopt_jk_ctx* ctx, const double* dH, const dou
 
 /* Tile and split tuning. The build divides the auxiliary index into Q-splits
  * (partial sums over Q ranges, added in FP64 at the end): params[6] =
- * {FP64/FP32/bf16 exchange splits, FP64 J splits (0: the fewest the kernel's
+ * {FP64/FP32/bf16 exchange splits (as create picked them, the count is that of
+ * the FP64 exchange and the FP32 and bf16 ones have their own; any other value
+ * holds for all three, the FP64 exchange using fewer where a split would have
+ * under 32 terms), FP64 J splits (0: the fewest the kernel's
  * gamma cache allows, at least 16), integer exchange splits, integer gamma
  * splits, integer J splits, and where the integer Coulomb
  * pair starts on its side stream: 0 after the half-transform, 1 gamma beside

@@ -559,9 +559,10 @@ struct nopt_jk_ctx {
   void* Xe = nullptr;
   size_t Xe_bytes = 0;
   int ntiles8 = 0, nsk8 = 0;  // 64x64 exchange tiles of the FP64 and integer paths; the integer path's Q-splits
-  // Q-splits of the FP32 and bf16 exchanges: as many blocks of their 128x128
-  // tiles as the FP64 exchange has of its own
-  int nsk128() const { return (int)std::max(1L, std::min(naux, (long)nsk * ntiles8 / ntiles)); }
+  // Q-splits of the FP32 and bf16 exchanges (tiles of 128x128): the caller's or
+  // the tuner's count as it is, and with the FP64 count that create picked their own
+  int nsk_create = 0, nsk128_create = 0;
+  int nsk128() const { return nsk == nsk_create ? nsk128_create : nsk; }
   // the lower triangle of B as packed rows in 16-column segments (N28 as
   // int32, then d4 as bytes: 5*splane bytes), read by the Coulomb pair and,
   // without bfull, by the half-transform; the segment and slot tables, gamma
@@ -1735,6 +1736,16 @@ int nopt_jk_create_ex(int device, long nbf, long naux, int flags, nopt_jk_ctx** 
     // 300, 487, 692 us with four, of 490 functions 3.15 against 3.01 ms
     c->nsk = (int)std::max(1L, std::min(naux, std::max(2L * ncu / c->ntiles8,
                                                        std::min(4L * ncu / c->ntiles8, naux / 64))));
+    c->nsk_create = c->nsk;
+    // FP32 and bf16 exchanges: as many blocks of their own tiles. With 512 blocks
+    // against 1024: 192 functions 256 and 277 us (FP32), 275 and 298 (BF16X3),
+    // 305 and 327 (BF16X6), 250 functions 393, 425, 466 and 417, 445, 485, 298
+    // functions 735, 730, 825 and 785, 750, 845; at 490 functions, where 1024 go
+    // out, 1000 took 3053, 3547, 4060 and 1040 3033, 3543, 4052
+    const long nt = c->ntiles;
+    c->nsk128_create =
+        (int)std::max(1L, std::min(naux, std::max((2L * ncu + nt - 1) / nt,
+                                                  std::min((4L * ncu + nt - 1) / nt, naux / 64 * c->ntiles8 / nt))));
     const long slots = 2L * ncu / 8;  // per XCD
     int best = 8;
     double best_eff = 0.0;

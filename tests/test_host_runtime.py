@@ -36,3 +36,7 @@ def test_device_bytes_are_those_held(run):
 
 def test_autotuner_leaves_unused_settings(run):
     run("host_autotune")
+
+
+def test_stored_exchange_splits_are_those_launched(run):
+    run("host_exchange_splits")
