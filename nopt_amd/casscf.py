@@ -283,20 +283,31 @@ class CASSCF:
 
     def run(self, C0, g_conv=1e-7, e_conv=1e-11, max_it=300, memory=10, trust=0.3, verbose=False):
         """L-BFGS over the non-redundant rotations from orbitals C0 (columns,
-        orthonormal in the overlap metric)."""
+        orthonormal in the overlap metric).
+
+        A step is kept when the energy falls. Builds that round coarsely (the
+        integer mode) leave a noise in the energy that is no smooth function of
+        the orbitals, about 1e-7 Eh for C2H4, more than a step changes it by near
+        the end, while the gradient is good to far below 1e-4: steps that lower the
+        gradient would then be refused for ever. So a step whose change of the
+        energy, by the slopes at its two ends, is below e_conv, the caller's own
+        resolution, is judged by the slopes (Hager and Zhang's approximate Wolfe
+        condition, SIAM J. Optim. 16, 170 (2005)), and where the energies at its
+        ends contradict the slopes by more than e_conv, the slopes' change is
+        the one that the convergence test looks at."""
         C = np.array(C0, dtype=np.float64)
         nmo = C.shape[1]
         msk = self.mask(nmo)
         r = self.evaluate(C)
         S_hist, Y_hist, hist = [], [], []
-        E_prev = None
+        change = None  # of the energy in the last step
         for it in range(max_it):
             g = r["grad"][msk]
             gmax = float(np.abs(g).max())
             hist.append((it, r["E"], gmax))
             if verbose:
                 print(f"CAS {it} E={r['E']:.12f} |g|max={gmax:.3e} trust={trust:.3f}")
-            if gmax < g_conv and E_prev is not None and abs(r["E"] - E_prev) < e_conv:
+            if gmax < g_conv and change is not None and change < e_conv:
                 r.update(C=C, iters=it, gmax=gmax, history=hist, converged=True)
                 return r
             f = np.diag(r["Ft_mo"])
@@ -325,12 +336,15 @@ class CASSCF:
             kap = kap - kap.T
             Cn = C @ sl.expm(kap)
             rn = self.evaluate(Cn)
-            if rn["E"] > r["E"] + 1e-12 * max(1.0, abs(r["E"])):
+            gn = rn["grad"][msk]
+            dE = rn["E"] - r["E"]
+            slopes = 0.5 * float(step @ (g + gn))
+            if dE > 1e-12 * max(1.0, abs(r["E"])) and not -e_conv < slopes < 0.0:
                 trust = max(0.5 * trust, 1e-4)
                 S_hist.clear()
                 Y_hist.clear()
                 continue
-            y = rn["grad"][msk] - g
+            y = gn - g
             if float(step @ y) > 1e-14:
                 S_hist.append(step)
                 Y_hist.append(y)
@@ -339,7 +353,7 @@ class CASSCF:
                     Y_hist.pop(0)
             if big <= trust:
                 trust = min(2.0 * trust, 1.0)
-            E_prev = r["E"]
+            change = abs(slopes) if abs(dE - slopes) > e_conv else abs(dE)
             C, r = Cn, rn
         r.update(C=C, iters=max_it, gmax=float(np.abs(r["grad"][msk]).max()), history=hist, converged=False)
         return r

@@ -28,9 +28,8 @@ class SCFResult(dict):
 def fix_signs(C):
     """C with each column's sign such that its first component within 1e-6 of
     its largest magnitude is positive. LAPACK's signs change with the rounding
-    of the matrix; what starts from these orbitals with a build that rounds as
-    coarsely as the integer mode (a CASSCF taken down to that mode's gradient
-    noise) goes another way for other signs, and should not for rounding."""
+    of the matrix, and with them the rounding of every integer build that starts
+    from these orbitals; a run should be the same run after either."""
     a = np.abs(C)
     first = (a > (1.0 - 1e-6) * a.max(axis=0)).argmax(axis=0)
     return C * np.where(C[first, np.arange(C.shape[1])] < 0.0, -1.0, 1.0)
