@@ -1410,7 +1410,7 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
                         f64 && fused ? nopt::kHalfF64Rows : 0, nsj, Jpart, (long)nsj * nn};
   const nopt::ItemJ ji8{c->Bs, c->splane, 16L * c->nseg, c->Be, nbf, naux, c->lsegs, c->nlseg,
                         nsb ? w.gslot : w.gamma, naux, Jpart, (long)nsj * nn, (c->nlseg + 255) / 256, nsj, 1};
-  // in line, the J pass goes into the launch of the first exchange
+  // in line, the J pass goes into the launch of the first exchange (jrides: there is one)
   bool jwait = false;
   auto coulomb_j = [&]() -> hipError_t {
     if (i8 && rec) {
@@ -1624,7 +1624,6 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
     HIPCHK(hipGetLastError());
   }
   mark(5);
-  if (jwait) HIPCHK(coulomb_j());  // there was no exchange
   if (coulomb_at == 2) HIPCHK(coulomb_out());
   if (overlap) {
     HIPCHK(hipEventRecord(c->ev_join, c->side));
