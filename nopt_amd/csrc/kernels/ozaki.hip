@@ -152,9 +152,9 @@ __global__ __launch_bounds__(256) void k_stage(StageList l) {
 // 3 writes the packed lower triangle Bs (planes = Bs, pstride = splane,
 // ld = sq) of the reordered functions: the element (m, n) goes to row
 // max(a, b), column min(a, b) with a, b = pinv[m], pinv[n], as digits5 of the
-// value at that row's exponent. With pinv, modes 1 and 2 write the row and
-// column pinv[m], pinv[n] as well (the function m of B is function pinv[m]
-// of the kept forms).
+// value at that row's exponent. With pinv, mode 2 writes the row and column
+// pinv[m], pinv[n] as well (the function m of B is function pinv[m] of the
+// kept forms).
 template <int MODE>
 __global__ __launch_bounds__(256) void k_packed_tiles(const double* __restrict__ A, long cp, int m0, int m1, int nbf,
                                                       double* __restrict__ out64, long ld,
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(256) void k_packed_tiles(const double* __restrict__
     } else if constexpr (MODE == 1) {
       double mx = fabs(v[k]);
       for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-      if (c == 0 && m < m1) atomicMax(rowmax + P * nbf + fn(m), (unsigned long long)__double_as_longlong(mx));
+      if (c == 0 && m < m1) atomicMax(rowmax + P * nbf + m, (unsigned long long)__double_as_longlong(mx));
     } else if constexpr (MODE == 2) {
       if (ok) {
         const long row = P * nbf + fn(m);
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void k_packed_tiles(const double* __restrict__
     } else if constexpr (MODE == 1) {
       double mx = fabs(x);
       for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-      if (c == 0 && n < nbf) atomicMax(rowmax + P * nbf + fn(n), (unsigned long long)__double_as_longlong(mx));
+      if (c == 0 && n < nbf) atomicMax(rowmax + P * nbf + n, (unsigned long long)__double_as_longlong(mx));
     } else if constexpr (MODE == 2) {
       if (ok) {
         const long row = P * nbf + fn(n);
@@ -241,7 +241,7 @@ __global__ void k_rowmax_exponent(const unsigned long long* __restrict__ rowmax,
                                   const int* __restrict__ pinv, int nbf) {
   const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= rows) return;
-  expo[pinv ? r / nbf * nbf + pinv[r % nbf] : r] = row_exponent(__longlong_as_double((long long)rowmax[r]));
+  expo[r / nbf * nbf + pinv[r % nbf]] = row_exponent(__longlong_as_double((long long)rowmax[r]));
 }
 
 // mx[p] = max(mx[p], max_r |A[r*w + p]|): a pair per thread, eight rows in flight
@@ -1535,10 +1535,10 @@ hipError_t unpack_packed_f64(const double* A, long cp, int m0, int m1, int nbf, 
 }
 
 hipError_t rowmax_packed(const double* A, long cp, int m0, int m1, int nbf, long naux, unsigned long long* rowmax,
-                         hipStream_t s, const int* pinv) {
+                         hipStream_t s) {
   if (!packed_chunk_ok(cp, m0, m1, nbf, naux)) return hipErrorInvalidValue;
   k_packed_tiles<1><<<packed_grid(m0, m1, naux), 256, 0, s>>>(A, cp, m0, m1, nbf, nullptr, 0, rowmax, nullptr, 0,
-                                                               nullptr, 0, pinv);
+                                                               nullptr, 0, nullptr);
   return hipGetLastError();
 }
 

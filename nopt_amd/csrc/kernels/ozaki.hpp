@@ -45,18 +45,17 @@ hipError_t launch_stage(StageList& l, hipStream_t s);
 // (n <= m) of every P < naux: each element goes to both full rows it belongs
 // to, (P, m) and (P, n). unpack_packed_f64 writes FP64 rows B[(P*nbf + r)*ld + col];
 // rowmax_packed folds the chunk into the row maxima (bit patterns, zeroed by
-// the caller), rowmax_exponents turns them into exponents, and
-// split_packed_i8 writes the digit planes of split_rows_i8 with those
-// exponents. Padding columns are the caller's to clear. With pinv, the
-// function m of the chunk is function pinv[m] of the rows written (rows and
-// columns both reordered).
+// the caller), rowmax_exponents turns them into exponents (row m of a function
+// of nbf rows to row pinv[m] of expo), and split_packed_i8 writes the digit
+// planes of split_rows_i8 with those exponents. Padding columns are the
+// caller's to clear. With pinv, the function m of the chunk is function pinv[m]
+// of the digit rows (rows and columns both reordered).
 hipError_t unpack_packed_f64(const double* A, long cp, int m0, int m1, int nbf, long naux, double* B, long ld,
                              hipStream_t s);
 hipError_t rowmax_packed(const double* A, long cp, int m0, int m1, int nbf, long naux, unsigned long long* rowmax,
-                         hipStream_t s, const int* pinv = nullptr);
-// (with pinv: row m of each function to row pinv[m] of expo, nbf rows a function)
-hipError_t rowmax_exponents(const unsigned long long* rowmax, long rows, int* expo, hipStream_t s,
-                            const int* pinv = nullptr, int nbf = 1);
+                         hipStream_t s);
+hipError_t rowmax_exponents(const unsigned long long* rowmax, long rows, int* expo, hipStream_t s, const int* pinv,
+                            int nbf);
 // mx[p] = max(mx[p], max over the rows of |A[r*w + p]|), p < w (NaNs left out)
 hipError_t pair_max(const double* A, long w, long rows, double* mx, hipStream_t s);
 hipError_t split_packed_i8(const double* A, long cp, int m0, int m1, int nbf, long naux, const int* expo, int ns,
