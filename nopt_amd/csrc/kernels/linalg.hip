@@ -115,7 +115,8 @@ __global__ __launch_bounds__(256, 4) void k_gemm_f64(GemmArgs p) {
 
 hipError_t launch_gemm(bool transB, int M, int N, int K, double alpha, const double* A, long lda, const double* B,
                        long ldb, double beta, double* C, long ldc, bool lower, hipStream_t s) {
-  if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
+  if (M <= 0 || N <= 0) return hipSuccess;
+  if (K <= 0) return hipErrorInvalidValue;
   const GemmArgs p{A, B, C, lda, ldb, ldc, M, N, K, alpha, beta, lower, (M + 63) / 64, (N + 63) / 64};
   if ((long)p.mt * p.nt > 0x7fffffffL) return hipErrorInvalidValue;
   if (transB)

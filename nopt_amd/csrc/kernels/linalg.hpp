@@ -4,7 +4,7 @@
 
 namespace nopt {
 // C = alpha * A * op(B) + beta * C; op(B) = B (K x N, ldb) or, with transB,
-// the transpose of B (N x K, ldb). Row-major.
+// the transpose of B (N x K, ldb). Row-major; K at least 1.
 hipError_t gemm_f64(bool transB, int M, int N, int K, double alpha, const double* A, long lda,
                     const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s);
 // In-place lower Cholesky A = L L^T (strict upper part zeroed); Xd gets the

@@ -40,3 +40,7 @@ def test_autotuner_leaves_unused_settings(run):
 
 def test_stored_exchange_splits_are_those_launched(run):
     run("host_exchange_splits")
+
+
+def test_matrix_product_over_no_terms_is_refused(run):
+    run("host_gemm_empty")
