@@ -540,6 +540,7 @@ struct nopt_jk_ctx {
   long xD_cap[kMaxBatch - 1] = {}, xC_cap[kMaxBatch - 1] = {}, xJ_cap[kMaxBatch - 1] = {},
        xK_cap[kMaxBatch - 1] = {};
   int* info = nullptr;
+  int* info_host = nullptr;  // pinned, so that info's copy does not hold up the host (made by the first set_B)
   // integer forms of B: the row exponents (Be, and as bytes Be8[Q*ld8 + n]),
   // the packed lower triangle Bs below, and, when bfull, the full rows as
   // four digit planes (4 x naux*nbf x ld8) for the half-transform; the
@@ -1855,6 +1856,7 @@ void nopt_jk_destroy(nopt_jk_ctx* c) {
   dev_free(c->act);
   free_ring(c);
   dev_free(c->info);
+  if (c->info_host) (void)hipHostFree(c->info_host);
   dev_free(c->Bd);
   dev_free(c->Be);
   dev_free(c->Be8);
@@ -2176,15 +2178,13 @@ int nopt_jk_set_B(nopt_jk_ctx* c, const double* eri3, const double* metric) {
   if (!rc) {
     hipError_t e = hipMemcpyAsync(dV, metric, sizeof(double) * na * na, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = nopt::cholesky_f64(dV, na, (int)na, dV + na * na, c->info, c->stream);
-    int* info = nullptr;  // pinned, so that its copy does not hold up the host
-    if (e == hipSuccess) e = hipHostMalloc((void**)&info, sizeof(int), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMemcpyAsync(info, c->info, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess && !c->info_host) e = hipHostMalloc((void**)&c->info_host, sizeof(int), hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMemcpyAsync(c->info_host, c->info, sizeof(int), hipMemcpyDeviceToHost, c->stream);
     if (e != hipSuccess)
       rc = set_error(NOPT_EHIP, std::string("metric factorisation: ") + hip_msg(e));
     else
-      rc = form_B(c, eri3, dV, dV + na * na, info);
+      rc = form_B(c, eri3, dV, dV + na * na, c->info_host);
     (void)hipStreamSynchronize(c->stream);
-    if (info) (void)hipHostFree(info);
   }
   dev_free(dV);
   return rc;

@@ -16,7 +16,7 @@ std::map<const void*, std::string>& kernels() {  // filled while the library loa
 }
 std::vector<Launch> launches;
 size_t live = 0;
-int mallocs = 0, fail_at = 0;
+int mallocs = 0, fail_at = 0, pinned = 0, pinned_live = 0;
 float elapsed = 1e6f;
 }  // namespace fake
 
@@ -62,8 +62,15 @@ int hipFree(void* p) {
   std::free(p);
   return kOk;
 }
-int hipHostMalloc(void** p, size_t bytes, unsigned) { return *p = std::calloc(bytes, 1), kOk; }
-int hipHostFree(void* p) { return std::free(p), kOk; }
+int hipHostMalloc(void** p, size_t bytes, unsigned) {
+  ++fake::pinned;
+  ++fake::pinned_live;
+  return *p = std::calloc(bytes, 1), kOk;
+}
+int hipHostFree(void* p) {
+  --fake::pinned_live;
+  return std::free(p), kOk;
+}
 int hipMemcpy(void* d, const void* s, size_t n, int) { return copy(d, s, n); }
 int hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) { return copy(d, s, n); }
 int hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, int, void*) {

@@ -19,6 +19,7 @@ struct Launch {
 extern std::vector<Launch> launches;  // kernels launched so far
 extern size_t live;                   // bytes allocated and not freed
 extern int mallocs, fail_at;          // allocations so far; the one that fails (0: none)
+extern int pinned, pinned_live;       // pinned host allocations so far, and those not freed
 }  // namespace fake
 
 #define EXPECT(cond)                                                          \

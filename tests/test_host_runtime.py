@@ -44,3 +44,7 @@ def test_stored_exchange_splits_are_those_launched(run):
 
 def test_matrix_product_over_no_terms_is_refused(run):
     run("host_gemm_empty")
+
+
+def test_pinned_memory_is_kept(run):
+    run("host_pinned")
