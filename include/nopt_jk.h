@@ -245,9 +245,11 @@ int nopt_jk_autotune(nopt_jk_ctx* ctx, const double* dD, const double* dC, long 
 /* Per-phase timing with HIP events on the build's stream (no counterpart in
  * NOPT, whose RHF loop disables its step timers, src/SCF.cpp:124). When
  * enabled, each build (or batch) records events around its six phases:
- * staging of D and C, half-transform (with the fused gamma partials of a
- * single FP64/FP32/bf16 build), gamma, J partials, exchange (K products and
- * K output) and the J output. read_timing returns the summed milliseconds per
+ * staging of D and C, half-transform (with the gamma partials of an FP64 build
+ * of one or two densities or an FP32/bf16 build of one), gamma (nothing in that
+ * FP64 build, whose J pass adds the partials), J partials, exchange (K products
+ * and K output) and the J output; the phases then run one after the other on
+ * the build's stream, also those that otherwise share a launch. read_timing returns the summed milliseconds per
  * phase (ms[6]) and the number of builds recorded since the last read, then
  * resets. */
 int nopt_jk_set_timing(nopt_jk_ctx* ctx, int enable);

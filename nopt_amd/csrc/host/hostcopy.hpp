@@ -6,7 +6,7 @@ namespace nopt {
 
 // dst[r*width ..] = src[r*pitch ..], `width` bytes of each of `rows` rows, by up
 // to four threads (one copies 36 to 42 GB/s into pinned memory, two 60, four
-// 100, more than the device takes from it).
+// 80 to 100, more than the device takes from it).
 void copy_rows(char* dst, const char* src, size_t width, size_t pitch, long rows);
 
 }  // namespace nopt

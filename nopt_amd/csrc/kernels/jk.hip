@@ -609,7 +609,7 @@ struct nopt_jk_ctx {
 
 namespace {
 // largest triangle of B (in FP64, times the densities) of which a build runs in
-// line on one stream (enqueue_batch): FP64 and integer builds whose J pass rides
+// line on one stream (route_of): FP64 and integer builds whose J pass rides
 // on the exchange's launch, and the others
 constexpr size_t kInlineF64 = (size_t)1 << 30, kInlineI8 = (size_t)288 << 20, kInlineOther = (size_t)64 << 20;
 constexpr int kPhases = 6;  // staging, half-transform, gamma, J partials, exchange, J output
@@ -838,14 +838,15 @@ int find_live(nopt_jk_ctx* c) {
 // 29 GB/s in one host thread, so larger transfers pass through two pinned
 // pieces, one filled by several threads while the other is on its way; the
 // context keeps the pieces. One copy at a time: with the next one queued behind
-// it the pair ran at 28 GB/s, so at 37. 303 MB take 8.3 ms (pieces of 16 MB
-// 7.9), 16.5 as one strided copy. Without the pieces (small transfers, no pinned
-// memory to be had) the runtime's own copy; and for the rest of a tensor once a
-// piece took kRingSlow seconds to fill (usually 0.15 ms): the process then has
-// more running threads than processors (a BLAS library's, still spinning after a
-// product), each of the copying threads can lose a time slice of some ms, and one
-// thread fares better: 589 MB right after a NumPy product took 98 ms, so 33 to 45
-// (22 with the processors free, 52 to 59 without pieces).
+// it the pair was slower. 303 MB take 6.7 ms, 46 GB/s (a piece is filled in 0.10
+// ms and takes 0.17 to copy, as the host sees it), 16.5 as one strided copy.
+// Without the pieces (small transfers, no pinned memory to be had) the runtime's
+// own copy; and for the rest of a tensor once a piece took kRingSlow seconds to
+// fill: the process then has more running threads than processors (a BLAS
+// library's, still spinning after a product), each of the copying threads can
+// lose a time slice of some ms, and one thread fares better: 589 MB right after a
+// NumPy product took 98 ms, so 33 to 45 (22 with the processors free, 52 to 59
+// without pieces).
 constexpr size_t kRingBytes = (size_t)8 << 20, kRingMin = (size_t)32 << 20;
 constexpr double kRingSlow = 1e-3;
 int upload_rows(nopt_jk_ctx* c, char* dst, const char* src, size_t width, size_t pitch, long rows, hipStream_t s) {
@@ -1188,10 +1189,10 @@ struct Rec {
 // into the launch of the first exchange, where it reads memory beside the matrix
 // products all the same. In line and with the second stream, microseconds, FP64:
 // 96 functions 44 and 59, 192 functions 156 and 172, 250 functions 329 and 345,
-// 346 functions 995 and 1015, 394 functions 1612 and 1625, 490 functions 3154
-// and 3000; int8: 96 functions 45 and 70, 192 functions 139 and 151, 240
-// functions 240 and 240, 288 functions 384 and 376; two densities cross at half
-// the triangle.
+// 346 functions (0.80 GB) 995 and 1015, 394 functions (1.18 GB, just above the
+// limit) 1612 and 1625, 490 functions (2.28 GB) 3154 and 3000; int8: 96 functions
+// 45 and 70, 192 functions 139 and 151, 240 functions (268 MB) 240 and 240, 288
+// functions (463 MB) 384 and 376; two densities cross at half the triangle.
 struct Route {
   int nsb = 0;
   bool jrides = false, inl = false;
@@ -1477,9 +1478,9 @@ int enqueue_batch(nopt_jk_ctx* c, int nd, const BuildItem* it, int prec, hipStre
       stage_rows<float>(w.Dp, ldb, 0, 0, (float*)w.Cp + ncol * ldb, ldb, tail, s);
   }
   HIPCHK(hipGetLastError());
-  // the integer Coulomb pair starts where cplace says (tuned: beside the
-  // half-transform it takes CUs from it, after it it shares the device with
-  // the exchange)
+  // the integer Coulomb pair of the second stream starts where cplace says
+  // (tuned: beside the half-transform it takes CUs from it, after it it shares
+  // the device with the exchange)
   if (overlap && !fused && !i8) {
     HIPCHK(hipEventRecord(c->ev_fork, s));
     HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));

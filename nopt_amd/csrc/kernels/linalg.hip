@@ -131,8 +131,9 @@ constexpr int NB = 64;
 
 // Factors the kb x kb diagonal block at (k0, k0) of A in place (lower, its
 // strict upper part zeroed) and writes the inverse of the factor, 64 x 64 with
-// the rows and columns beyond kb those of a unit matrix, to Xd. One block of four waves; the 64 x 64 block lives in LDS as
-// 4 x 4 blocks of 16 (rows and columns beyond kb those of a unit matrix). A
+// the rows and columns beyond kb those of a unit matrix, to Xd. One block of
+// four waves; the 64 x 64 block lives in LDS as 4 x 4 blocks of 16 (rows and
+// columns beyond kb those of a unit matrix). A
 // panel of 16 columns is factored by one wave with a row per lane and the
 // columns in registers (pivot and row values by lane reads), the blocks right
 // of it are updated on the matrix cores. The inverse starts from those of the
